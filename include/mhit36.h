@@ -286,8 +286,7 @@ int mhit_energy_spectrum(mhit_ctx* ctx, int32_t nbins, double* E, int32_t* nshel
  * process ends; min(nbins, shells) above that limit returns MHIT_ERR_ARG.
  * Every call on a device shares its array: calls that overlap on one
  * device (from several threads or contexts) race.  Results as
- * mhit_energy_spectrum's (the shell sums are atomic adds, so the two agree
- * to rounding, not bit for bit).                                          */
+ * mhit_energy_spectrum's.                                                 */
 #define MHIT_SPECTRUM_NOALLOC_MAX_BINS 4096
 int mhit_energy_spectrum_noalloc(mhit_ctx* ctx, int32_t nbins, double* E, int32_t* nshells);
 

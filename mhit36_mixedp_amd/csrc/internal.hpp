@@ -265,6 +265,11 @@ int launch_ns_march(mhit_ctx* c);
 int launch_acdi_march_batch(mhit_ctx* const* boxes, int nb, ArgArena& arena, hipStream_t st);
 int launch_ns_march_batch(mhit_ctx* const* boxes, int nb, ArgArena& arena, hipStream_t st);
 
+// spectra.hip: shells that the transform of an n^3 box fills, and workgroups
+// of the shell sums, whose partials are kept in the diagnostics' partials
+int shells_used(int n);
+int spectrum_blocks(int n);
+
 // tracers.hip
 int launch_tracers(mhit_ctx* c, hipStream_t st);
 int sort_tracers(mhit_ctx* c);          // stable cell-order permutation
