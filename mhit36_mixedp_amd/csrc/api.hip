@@ -546,7 +546,7 @@ int mhit_destroy(mhit_ctx* c) {
                     c->phi, c->phi_next, c->rhsphi, c->rhsphi_o, c->psi, c->tanh_psi, c->normx, c->normy,
                     c->normz, c->fxst, c->fyst, c->fzst, c->pres, c->spec, c->nyq, c->tw, c->kk,
                     c->mysin, c->partials, c->dpartials, c->S, c->ptag, c->px, c->py, c->pz,
-                    c->pu1, c->pv1, c->pw1};
+                    c->pu1, c->pv1, c->pw1, c->drop_buf};
     dump_release(c);   // waits for a dump still being written
     clear_graphs(c);
     for (void* p : ptrs) dfree(p);

@@ -65,6 +65,7 @@ struct mhit_ctx {
     void* sort_tmp = nullptr;
     size_t sort_tmp_bytes = 0;
     int64_t sort_cap = 0;
+    double* drop_buf = nullptr;   // drop statistics: tables, list and sums (drops.hip)
     // host copy of scalars after the last sync
     mhit::DevScalars S_host{};
     // captured timesteps, keyed by the buffers they use (phi ping-pong
