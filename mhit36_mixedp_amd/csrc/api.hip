@@ -485,7 +485,7 @@ int mhit_create(const mhit_params* P, mhit_ctx** out) {
     c->npart_blocks = correct_block_count(n);
     if ((rc = dmalloc(&c->partials, (size_t)c->npart_blocks * 6))) return fail(rc);
     c->ndiag_blocks = diag_block_count(n);
-    const size_t ndp = std::max((size_t)c->ndiag_blocks * 8, (size_t)spectrum_blocks(n) * shells_used(n));
+    const size_t ndp = std::max((size_t)(c->ndiag_blocks + 1) * 8, (size_t)spectrum_blocks(n) * shells_used(n));
     if ((rc = dmalloc(&c->dpartials, ndp))) return fail(rc);
     if ((rc = dmalloc(&c->S, 1))) return fail(rc);
 

@@ -242,7 +242,6 @@ int launch_ns(mhit_ctx* c) {
 // plane's p with a one-point halo at -x and -y is staged in LDS, and the
 // next plane is fetched into registers during the update.  The number of partials is
 // fixed by the grid, so the reduction order is deterministic.
-constexpr int kCorrZ = 16;                    // z split of the diagnostics pass
 constexpr int CO_NT = 512;                    // threads per workgroup
 // tile columns: 64, or 32 where n is not a multiple of 64 (96^3: a
 // 64-column tile would leave a third of the threads without a cell); rows
@@ -437,8 +436,15 @@ int correct_block_count(int n) {
     return (int)(g.x * g.y * g.z);
 }
 
+// Diagnostics: 64 x 8 columns per workgroup, chunks of 32 planes from
+// 512^3, 16 from 256^3 and 4 below (each chunk reads two planes more; short
+// chunks keep small boxes on all CUs).
+constexpr int DI_MY = 8;
+static int diag_zc(int n) { return n >= 512 ? 32 : n >= 256 ? 16 : 4; }
+static dim3 diag_grid(int n) { return dim3(div_up(n, 64), div_up(n, DI_MY), div_up(n, diag_zc(n))); }
 int diag_block_count(int n) {
-    return div_up(n, 64) * div_up(n, 4) * (kCorrZ < n ? kCorrZ : n);
+    const dim3 g = diag_grid(n);
+    return (int)(g.x * g.y * g.z);
 }
 
 // Finalize: means (main.f90:964-974), signed max after the mean removal
@@ -529,57 +535,75 @@ int launch_finalize_batch(mhit_ctx* const* boxes, int nb, ArgArena& arena, hipSt
 // KE, dissipation 2 nu <S_ij S_ij> with central differences
 // (post/compute_diss/main.f90:72-117, dx = lx/n, nu = mu/rho), max |D.u|
 // with the divergence stencil of main.f90:841-843, phi mass and range.
-__global__ __launch_bounds__(256)
+// A thread marches its column up a chunk of planes with the column's three
+// planes in registers; the x and y neighbours come from L1 and L2, so u, v,
+// w and phi cross HBM about once.  (With a thread's planes n/16 apart, all
+// neighbours from the caches and the partial sums added up on the host it
+// took 0.265 ms at 256^3 with phi and 0.07 ms to read them back; now 0.201
+// and 0.006 ms, 2.4 -> 1.4 ms a call at 512^3.  What is left is the latency
+// of 19 loads per plane and column at six waves per SIMD.)
+constexpr int NF = 8;
+// sums; fields 2 and 6 maxima, 5 the minimum
+__device__ __forceinline__ double diag_join(int f, double a, double b) {
+    return (f == 2 || f == 6) ? fmax(a, b) : (f == 5 ? fmin(a, b) : a + b);
+}
+__device__ __forceinline__ double diag_start(int f) {
+    return f == 5 ? INFINITY : (f == 6 ? -INFINITY : 0.0);
+}
+
+__global__ __launch_bounds__(64 * DI_MY)
 void k_diag(const double* __restrict__ u, const double* __restrict__ v,
             const double* __restrict__ w, const double* __restrict__ phi,
-            double* __restrict__ partials, Grid g, const DevScalars* __restrict__ S) {
-    constexpr int NF = 8;
-    __shared__ double red[NF][4];
+            double* __restrict__ partials, Grid g, int zc, const DevScalars* __restrict__ S) {
+    __shared__ double red[NF][DI_MY];
     const int n = g.n;
-    const int i = blockIdx.x * 64 + threadIdx.x;
-    const int j = blockIdx.y * 4 + threadIdx.y;
-    double acc[NF] = {0.0, 0.0, 0.0, 0.0, 0.0, INFINITY, -INFINITY, 0.0};
+    const Blk blk = launch_blk(1);
+    int tbx, tby, tbz;
+    xcd_tile(tbx, tby, tbz, blk);   // neighbouring tiles' halo rows from the same L2
+    const int i = tbx * 64 + threadIdx.x;
+    const int j = tby * DI_MY + threadIdx.y;
+    const int z0 = tbz * zc, z1 = min(z0 + zc, n);
+    double acc[NF];
+    for (int f = 0; f < NF; f++) acc[f] = diag_start(f);
     if (i < n && j < n) {
         const double m0 = S->mean[0], m1 = S->mean[1], m2 = S->mean[2];
-        const int ip = wrap_p(i, n), im = wrap_m(i, n), jp = wrap_p(j, n), jm = wrap_m(j, n);
+        // in-plane offsets; the deferred mean cancels in every difference
+        const int o = j * n + i, oxp = j * n + wrap_p(i, n), oxm = j * n + wrap_m(i, n);
+        const int oyp = wrap_p(j, n) * n + i, oym = wrap_m(j, n) * n + i;
+        const size_t plane = (size_t)n * n;
         const double h = 0.5 * g.dxi;
-        for (int k = blockIdx.z; k < n; k += gridDim.z) {
-            const int kp = wrap_p(k, n), km = wrap_m(k, n);
-            const size_t q = idx3(i, j, k, n);
-#define U(a, b, c) (u[idx3(a, b, c, n)] - m0)
-#define V(a, b, c) (v[idx3(a, b, c, n)] - m1)
-#define W(a, b, c) (w[idx3(a, b, c, n)] - m2)
-            const double uu = U(i, j, k), vv = V(i, j, k), ww = W(i, j, k);
-            if (!isfinite(uu) || !isfinite(vv) || !isfinite(ww)) acc[7] += 1.0;
-            acc[0] += uu * uu + vv * vv + ww * ww;
-            const double dudx = (U(ip, j, k) - U(im, j, k)) * h, dudy = (U(i, jp, k) - U(i, jm, k)) * h;
-            const double dudz = (U(i, j, kp) - U(i, j, km)) * h;
-            const double dvdx = (V(ip, j, k) - V(im, j, k)) * h, dvdy = (V(i, jp, k) - V(i, jm, k)) * h;
-            const double dvdz = (V(i, j, kp) - V(i, j, km)) * h;
-            const double dwdx = (W(ip, j, k) - W(im, j, k)) * h, dwdy = (W(i, jp, k) - W(i, jm, k)) * h;
-            const double dwdz = (W(i, j, kp) - W(i, j, km)) * h;
+        const size_t km = wrap_m(z0, n) * plane, k0 = z0 * plane;
+        double um = u[km + o], vm = v[km + o], wm = w[km + o];
+        double uu = u[k0 + o], vv = v[k0 + o], ww = w[k0 + o];
+        for (int k = z0; k < z1; k++) {
+            const double *U = u + k * plane, *V = v + k * plane, *W = w + k * plane;
+            const size_t kp = wrap_p(k, n) * plane;
+            const double up = u[kp + o], vp = v[kp + o], wp = w[kp + o];
+            const double uxp = U[oxp], vyp = V[oyp];
+            const double uc = uu - m0, vc = vv - m1, wc = ww - m2;
+            if (!isfinite(uc) || !isfinite(vc) || !isfinite(wc)) acc[7] += 1.0;
+            acc[0] += uc * uc + vc * vc + wc * wc;
+            const double dudx = (uxp - U[oxm]) * h, dudy = (U[oyp] - U[oym]) * h, dudz = (up - um) * h;
+            const double dvdx = (V[oxp] - V[oxm]) * h, dvdy = (vyp - V[oym]) * h, dvdz = (vp - vm) * h;
+            const double dwdx = (W[oxp] - W[oxm]) * h, dwdy = (W[oyp] - W[oym]) * h, dwdz = (wp - wm) * h;
             const double S12 = 0.5 * (dudy + dvdx), S13 = 0.5 * (dudz + dwdx), S23 = 0.5 * (dvdz + dwdy);
             acc[1] += dudx * dudx + dvdy * dvdy + dwdz * dwdz + 2.0 * (S12 * S12 + S13 * S13 + S23 * S23);
-            const double dv = ((U(ip, j, k) - uu) + (V(i, jp, k) - vv) + (W(i, j, kp) - ww)) * g.dxi;
-#undef U
-#undef V
-#undef W
+            const double dv = ((uxp - uu) + (vyp - vv) + (wp - ww)) * g.dxi;
             acc[2] = fmax(acc[2], fabs(dv));
             if (phi) {
-                const double ph = phi[q];
+                const double ph = phi[k * plane + o];
                 if (!isfinite(ph)) acc[7] += 1.0;
                 acc[3] += ph;
                 acc[5] = fmin(acc[5], ph);
                 acc[6] = fmax(acc[6], ph);
             }
+            um = uu; vm = vv; wm = ww;
+            uu = up; vv = vp; ww = wp;
         }
     }
     for (int f = 0; f < NF; f++) {
         double x = acc[f];
-        for (int off = 32; off > 0; off >>= 1) {
-            const double y = __shfl_xor(x, off, 64);
-            x = (f == 2 || f == 6) ? fmax(x, y) : (f == 5 ? fmin(x, y) : x + y);
-        }
+        for (int off = 32; off > 0; off >>= 1) x = diag_join(f, x, __shfl_xor(x, off, 64));
         acc[f] = x;
     }
     if ((threadIdx.x & 63) == 0)
@@ -588,10 +612,25 @@ void k_diag(const double* __restrict__ u, const double* __restrict__ v,
     if (threadIdx.y == 0 && threadIdx.x < NF) {
         const int f = threadIdx.x;
         double r = red[f][0];
-        for (int t = 1; t < 4; t++)
-            r = (f == 2 || f == 6) ? fmax(r, red[f][t]) : (f == 5 ? fmin(r, red[f][t]) : r + red[f][t]);
-        const size_t b = ((size_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+        for (int t = 1; t < DI_MY; t++) r = diag_join(f, r, red[f][t]);
+        const size_t b = ((size_t)tbz * blk.ny + tby) * blk.nx + tbx;
         partials[b * NF + f] = r;
+    }
+}
+
+// The workgroups' partials to out[0, NF), a workgroup per field.
+__global__ __launch_bounds__(1024)
+void k_diag_sum(const double* __restrict__ partials, int nb, double* __restrict__ out) {
+    __shared__ double red[16];
+    const int t = threadIdx.x, f = blockIdx.x;
+    double r = diag_start(f);
+    for (int b = t; b < nb; b += 1024) r = diag_join(f, r, partials[(size_t)b * NF + f]);
+    for (int off = 32; off > 0; off >>= 1) r = diag_join(f, r, __shfl_xor(r, off, 64));
+    if ((t & 63) == 0) red[t >> 6] = r;
+    __syncthreads();
+    if (t == 0) {
+        for (int v = 1; v < 16; v++) r = diag_join(f, r, red[v]);
+        out[f] = r;
     }
 }
 
@@ -645,23 +684,13 @@ int launch_stream_probe(mhit_ctx* c, const double* const* in, int R, double* con
 }
 
 int launch_diag(mhit_ctx* c, double* out) {
-    const int n = c->n;
-    dim3 grid(div_up(n, 64), div_up(n, 4), kCorrZ < n ? kCorrZ : n), block(64, 4, 1);
-    k_diag<<<grid, block, 0, c->stream>>>(c->u, c->v, c->w, c->P.phiflag ? c->phi : nullptr,
-                                          c->dpartials, c->g, c->S);
+    const int nb = c->ndiag_blocks;
+    double* sum = c->dpartials + (size_t)nb * NF;
+    k_diag<<<diag_grid(c->n), dim3(64, DI_MY, 1), 0, c->stream>>>(
+        c->u, c->v, c->w, c->P.phiflag ? c->phi : nullptr, c->dpartials, c->g, diag_zc(c->n), c->S);
+    k_diag_sum<<<NF, 1024, 0, c->stream>>>(c->dpartials, nb, sum);
     MHIT_HIP_TRY(hipGetLastError());
-    const int nb = grid.x * grid.y * grid.z;
-    std::vector<double> h((size_t)nb * 8);
-    MHIT_HIP_TRY(hipMemcpyAsync(h.data(), c->dpartials, h.size() * sizeof(double),
-                                hipMemcpyDeviceToHost, c->stream));
-    MHIT_HIP_TRY(hipStreamSynchronize(c->stream));
-    double r[8] = {0.0, 0.0, 0.0, 0.0, 0.0, INFINITY, -INFINITY, 0.0};
-    for (int b = 0; b < nb; b++)
-        for (int f = 0; f < 8; f++) {
-            const double x = h[(size_t)b * 8 + f];
-            r[f] = (f == 2 || f == 6) ? std::fmax(r[f], x) : (f == 5 ? std::fmin(r[f], x) : r[f] + x);
-        }
-    for (int f = 0; f < 8; f++) out[f] = r[f];
+    MHIT_HIP_TRY(copy_on_stream(c, out, sum, NF * sizeof(double), hipMemcpyDeviceToHost));
     return MHIT_OK;
 }
 
