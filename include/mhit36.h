@@ -192,7 +192,8 @@ int mhit_set_ab2_state(mhit_ctx* ctx, double alpha, double beta, double gumax);
  * (fft_wave, and widths that move a pass to or from eight columns), which
  * changes rounding.                                                       */
 typedef struct mhit_tuning {
-    int32_t ns_mz;        /* z planes per workgroup, fused NS pass          */
+    int32_t ns_mz;        /* z planes per workgroup, fused NS pass (fewer in
+                             a launch that would leave CUs without one)     */
     int32_t ac_mz;        /* z planes per workgroup, fused ACDI pass        */
     int32_t xcd;          /* 1: XCD-aware workgroup order, fused passes (the
                              default up to 256^3 and in ensembles)          */

@@ -104,14 +104,36 @@ static void parse_tuning(const char* s, Tuning& t) {
     }
 }
 
+// Planes per workgroup of a marching pass over `tiles` tiles with `slots`
+// workgroups resident at once, at most cap.  The chunks run in rounds of
+// `slots`, and each costs its planes plus about four for the planes before
+// and after it, so rounds x (planes + 4) is what the last workgroup waits
+// for; the longest of equal choices has the least halo.
+int chunk_planes(int n, long long tiles, int slots, int cap) {
+    int best = 1;
+    long long cost = -1;
+    for (int c = 1; c <= n; c++) {
+        const int zc = div_up(n, c);
+        if (zc > cap) continue;
+        const long long t = (tiles * div_up(n, zc) + slots - 1) / slots * (zc + 4);
+        if (cost < 0 || t < cost) { cost = t; best = zc; }
+    }
+    return best;
+}
+
 // Launch shapes by grid size, then MHIT_TUNE; mhit_autotune refines.
-// A box alone: 64x8 tiles up to 64^3, 64x16 above (less halo); z chunks
-// of min(128, n/4) planes, halved (never below 4) until the NS pass has a
-// workgroup per CU.  Measured, ms per step, FP32 Poisson, single phase /
-// multiphase: 64^3 0.075 / 0.113 at 8 planes -> 0.066 / 0.091 at 4;
-// 128^3 0.137 / 0.206 at 16 planes (64x8 ACDI tiles) -> 0.124 / 0.175 at
-// 8; 256^3 0.700 / 1.021 at 32 -> 0.674 / 0.983 at 64; 512^3 keeps 128
-// (fewer warm-up planes than 64: 8.17 -> 8.07 ms).  Boxes batched in an
+// A box alone: 64 x 8 tiles up to 64^3, 64 x 16 above (less halo), and
+// 64 x 8 in the ACDI pass of 128^3 to 384^3, two workgroups to a CU (192^3
+// 0.468 -> 0.460 ms per step, 384^3 3.14 -> 3.11; 512^3 6.95 -> 6.98, so
+// not there); z chunks by chunk_planes.  Measured, ms per step, FP32
+// Poisson, single phase / multiphase, against chunks halved from
+// min(128, n/4) until there is a workgroup per CU: 96^3 0.081 / 0.114 at 6
+// planes -> 0.075 / 0.099 at 4 (240 instead of 160 workgroups); 192^3
+// 0.384 / 0.609 at 24 -> 0.325 / 0.460 at 28 (252 workgroups in one round
+// instead of 288 in two); 384^3 2.38 / 3.60 at 96 -> 2.16 / 3.11 at 55 (3.9
+// rounds instead of 2.25); 128^3 (8) and 256^3 (64) unchanged; 512^3 6.99
+// -> 6.97 at 256.  Launches that still leave CUs idle at 4 planes are
+// shortened further (pass_chunk in march.hip).  Boxes batched in an
 // ensemble: 64x16 tiles and min(n, 128) planes, which the ensemble then
 // shortens until its launches fill the GPU.
 void default_tuning(mhit_ctx* c, bool batched, bool env) {
@@ -123,20 +145,17 @@ void default_tuning(mhit_ctx* c, bool batched, bool env) {
     // 19.13-19.19k box-steps/s, 16 x 96^3 alone 19.0k -> 19.6k
     const int rows = (n > 64 && n % 64 != 0 && n % 96 == 0) ? 10
                    : (n > 64 && n % 64 != 0 && n % 32 == 0) ? 32 : ((!batched && n <= 64) ? 8 : 16);
-    int zc = std::min(128, n);
-    if (!batched) {
-        int cus = 0;
-        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess ||
-            cus <= 0)
-            cus = 256;
-        zc = std::min(128, std::max(4, n / 4));
-        const long long tiles = (long long)div_up(n, tile_cols(rows)) * div_up(n, rows);
-        while (tiles * div_up(n, zc) < cus && zc / 2 >= 4) zc /= 2;
-    }
-    c->tune.ns_mz = zc;
-    c->tune.ac_mz = zc;
     c->tune.ns_my = rows;
     c->tune.ac_my = rows;
+    c->tune.ns_mz = c->tune.ac_mz = std::min(128, n);
+    if (!batched) {
+        if (rows == 16 && n >= 128 && n < 512) c->tune.ac_my = 8;
+        auto tiles = [&](int my) { return (long long)div_up(n, tile_cols(my)) * div_up(n, my); };
+        const int ac_slots = (c->tune.ac_my == 8 && n > 64) ? 2 * c->cus : c->cus;
+        const int least = std::min(4, n);
+        c->tune.ns_mz = std::max(least, chunk_planes(n, tiles(rows), c->cus, 256));
+        c->tune.ac_mz = std::max(least, chunk_planes(n, tiles(c->tune.ac_my), ac_slots, 256));
+    }
     // XCD tile order: neighbouring tiles of a box then share an XCD's L2.
     // Batched (the 64^3 / 96^3 / 128^3 ensemble 18.78-18.84k -> 18.87-
     // 18.96k box-steps/s) and a box alone up to 256^3 (ms per step: 64^3
@@ -451,6 +470,9 @@ int mhit_create(const mhit_params* P, mhit_ctx** out) {
 
     auto fail = [&](int code) { mhit_destroy(c); return code; };
     if (hipGetDevice(&c->device) != hipSuccess) { set_error("hipGetDevice failed"); return fail(MHIT_ERR_HIP); }
+    if (hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess ||
+        c->cus <= 0)
+        c->cus = 256;
     default_tuning(c, false);   // launch shapes for this device's CU count
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
         set_error("hipStreamCreate failed");

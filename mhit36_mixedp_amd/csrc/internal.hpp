@@ -17,7 +17,7 @@ struct mhit_ctx {
     int n = 0;
     size_t N3 = 0;
     mhit::Grid g{};
-    int device = 0;
+    int device = 0, cus = 256;    // compute units of the device
     hipStream_t stream = nullptr;
     bool fp32 = true;
 
@@ -205,6 +205,9 @@ double* state_field(mhit_ctx* c, int fieldn);
 // ensemble), then the MHIT_TUNE overrides
 void default_tuning(mhit_ctx* c, bool batched, bool env = true);
 void tuning_env(mhit_ctx* c);   // the MHIT_TUNE overrides alone
+// api.hip: planes per workgroup (at most cap) of a marching pass over
+// `tiles` tiles, `slots` workgroups resident at once
+int chunk_planes(int n, long long tiles, int slots, int cap);
 // dump.hip: wait for a pending dump and free its buffers
 void dump_release(mhit_ctx* c);
 

@@ -141,34 +141,34 @@ void k_ns_march(NsArgs<TD> one, const NsArgs<TD>* __restrict__ tab, int nbox) {
             poff[t] = (e < H2 * W2) ? wrapn(j0 - 2 + ly, n) * n + wrapn(i0 - 2 + lx, n) : 0;
         }
     }
-    double pu[NV], pv[NV], pw[NV], pp[NPH];
-    auto fetch = [&](int k) {
+    struct Plane { double u[NV], v[NV], w[NV], p[PHI ? NPH : 1]; };
+    auto fetch = [&](int k, Plane& r) {
         const size_t base = (size_t)wrapn(k, n) * plane;
 #pragma unroll
         for (int t = 0; t < NV; t++) {
             if ((H1 * W1) % NT == 0 || tid + t * NT < H1 * W1) {
                 const size_t q = base + voff[t];
-                pu[t] = u[q]; pv[t] = v[q]; pw[t] = w[q];
+                r.u[t] = u[q]; r.v[t] = v[q]; r.w[t] = w[q];
             }
         }
         if (PHI) {
 #pragma unroll
             for (int t = 0; t < NPH; t++)
-                if ((H2 * W2) % NT == 0 || tid + t * NT < H2 * W2) pp[t] = phi[base + poff[t]];
+                if ((H2 * W2) % NT == 0 || tid + t * NT < H2 * W2) r.p[t] = phi[base + poff[t]];
         }
     };
-    auto commit = [&](int k) {
+    auto commit = [&](int k, const Plane& r) {
         const int s = ring3(k);
 #pragma unroll
         for (int t = 0; t < NV; t++) {
             const int e = tid + t * NT;
-            if (e < H1 * W1) { su[s][e] = pu[t] - m0; sv[s][e] = pv[t] - m1; sw[s][e] = pw[t] - m2; }
+            if (e < H1 * W1) { su[s][e] = r.u[t] - m0; sv[s][e] = r.v[t] - m1; sw[s][e] = r.w[t] - m2; }
         }
         if (PHI) {
 #pragma unroll
             for (int t = 0; t < NPH; t++) {
                 const int e = tid + t * NT;
-                if (e < H2 * W2) sp[s][e] = pp[t];
+                if (e < H2 * W2) sp[s][e] = r.p[t];
             }
         }
     };
@@ -244,18 +244,23 @@ void k_ns_march(NsArgs<TD> one, const NsArgs<TD>* __restrict__ tab, int nbox) {
 
     double fz_prev = 0.0, fz_cur = 0.0;
     // warm-up: planes z0-1, z0 of u,v,w; phi planes z0-2..z0 and fz(z0-1)
-    if (PHI) {
-        fetch(z0 - 2);
-        commit(z0 - 2);   // also fills the velocity slot of z0-2 = z0+1, rewritten below
+    // (the first planes in flight together: a chunk waits once for them)
+    Plane nx;
+    {
+        Plane r1, r0;
+        if (PHI) fetch(z0 - 2, nx);   // also fills the velocity slot of z0-2 = z0+1, rewritten below
+        fetch(z0 - 1, r1);
+        fetch(z0, r0);
+        if (PHI) commit(z0 - 2, nx);
+        fetch(z0 + 1, nx);
+        commit(z0 - 1, r1);
+        commit(z0, r0);
     }
-    fetch(z0 - 1);
-    commit(z0 - 1);
-    fetch(z0);
-    commit(z0);
     lds_sync();
-    if (PHI) fz_prev = sig6 * chem(z0 - 1, tx, ty) * 0.5 * (P(z0, tx, ty) - P(z0 - 2, tx, ty)) * dxi;
-    lds_sync();
-    fetch(z0 + 1);
+    if (PHI) {
+        fz_prev = sig6 * chem(z0 - 1, tx, ty) * 0.5 * (P(z0, tx, ty) - P(z0 - 2, tx, ty)) * dxi;
+        lds_sync();
+    }
 
     double dprev = 0.0, wsprev = 0.0;   // divergence partial and w* of the previous plane
     for (int k = z0; k <= z1; k++) {
@@ -270,7 +275,7 @@ void k_ns_march(NsArgs<TD> one, const NsArgs<TD>* __restrict__ tab, int nbox) {
         // y = MY (wave 1)
         const bool xedge = tid < MY, yedge = tid >= 64 && tid < 64 + MX;
         const int eb = tid, ea = tid - 64;
-        commit(k + 1);
+        commit(k + 1, nx);
         lds_sync();
         if (PHI) {
             // S1 at plane k: fx on x = -1..MX, fy on y = -1..MY, fz on the column
@@ -293,7 +298,7 @@ void k_ns_march(NsArgs<TD> one, const NsArgs<TD>* __restrict__ tab, int nbox) {
             }
             lds_sync();
         }
-        if (k + 2 <= z1 + 1) fetch(k + 2);   // next plane in flight during the compute
+        if (k + 2 <= z1 + 1) fetch(k + 2, nx);   // next plane in flight during the compute
         const int sm = ring3(k - 1), sc = ring3(k), sq = ring3(k + 1);
         const int c = at(tx, ty);
         const double rw = rhs_w(sm, sc, sq, fz_prev, fz_cur);
@@ -406,22 +411,22 @@ void k_acdi_march(AcdiArgs one, const AcdiArgs* __restrict__ tab, int nbox) {
         const int lx = e % W2, ly = e / W2;
         poff[t] = (e < H2 * W2) ? wrapn(j0 - 2 + ly, n) * n + wrapn(i0 - 2 + lx, n) : 0;
     }
-    double pf[NPL];
-    auto fetch = [&](int k) {
+    struct Plane { double p[NPL]; };
+    auto fetch = [&](int k, Plane& r) {
         const MHIT_GLOBAL double* __restrict__ pl = phi + (size_t)wrapn(k, n) * plane;
 #pragma unroll
         for (int t = 0; t < NPL; t++)
-            if ((H2 * W2) % NT == 0 || tid + t * NT < H2 * W2) pf[t] = pl[poff[t]];
+            if ((H2 * W2) % NT == 0 || tid + t * NT < H2 * W2) r.p[t] = pl[poff[t]];
     };
     // registers -> psi ring (halo 2) and phi ring (halo 1), main.f90:522-534
-    auto commit = [&](int k) {
+    auto commit = [&](int k, const Plane& r) {
         const int sps = ring3(k), sph = ring4(k);
 #pragma unroll
         for (int t = 0; t < NPL; t++) {
             const int e = tid + t * NT;
             if (e >= H2 * W2) break;
             const int lx = e % W2, ly = e / W2;
-            const double ph = pf[t];
+            const double ph = r.p[t];
             const double val = fmin(ph, 1.0);
             spsi[sps][e] = eps * ln_ratio(val + enm, 1.0 - val + enm);
             if (lx >= 1 && lx <= MX + 2 && ly >= 1 && ly <= MY + 2)
@@ -482,24 +487,31 @@ void k_acdi_march(AcdiArgs one, const AcdiArgs* __restrict__ tab, int nbox) {
         return fz;
     };
 
-    // warm-up: psi planes z0-2..z0 -> Fz(z0-1); plane z0+1 -> fluxes of z0
-    for (int k = z0 - 2; k <= z0; k++) {
-        fetch(k);
-        commit(k);
-    }
-    lds_sync();
     double fz_m1 = 0.0, fz_0 = 0.0, fz_p1 = 0.0;
+    // warm-up: psi planes z0-2..z0 -> Fz(z0-1); plane z0+1 -> fluxes of z0
+    // (all in flight together)
+    Plane nx;
     {
-        double fx, fy;
-        flux(z0 - 1, tx, ty, fx, fy, fz_m1);
+        Plane r2, r1, r0, rp;
+        fetch(z0 - 2, r2);
+        fetch(z0 - 1, r1);
+        fetch(z0, r0);
+        fetch(z0 + 1, rp);
+        fetch(z0 + 2, nx);
+        commit(z0 - 2, r2);
+        commit(z0 - 1, r1);
+        commit(z0, r0);
+        lds_sync();
+        {
+            double fx, fy;
+            flux(z0 - 1, tx, ty, fx, fy, fz_m1);
+        }
+        lds_sync();
+        commit(z0 + 1, rp);
     }
-    lds_sync();
-    fetch(z0 + 1);
-    commit(z0 + 1);
     lds_sync();
     int bf = 0;
     fz_0 = fluxes(z0, bf);
-    fetch(z0 + 2);
     lds_sync();
 
     double wk = 0.0;
@@ -516,9 +528,9 @@ void k_acdi_march(AcdiArgs one, const AcdiArgs* __restrict__ tab, int nbox) {
             wp = w[idx3(i, j, wrap_p(k, n), n)] - m2;
             ro = rphi_o[q];
         }
-        commit(k + 2);
+        commit(k + 2, nx);
         lds_sync();
-        if (k + 3 <= z1 + 1) fetch(k + 3);   // next plane in flight during the compute
+        if (k + 3 <= z1 + 1) fetch(k + 3, nx);   // next plane in flight during the compute
         fz_p1 = fluxes(k + 1, bf ^ 1);
         if (live) {
             const double pc = PH(k, tx, ty);
@@ -552,8 +564,18 @@ void k_acdi_march(AcdiArgs one, const AcdiArgs* __restrict__ tab, int nbox) {
 }
 
 // ------------------------------------------------------------- launchers
+// z chunk of a launch over nb boxes: the tuned one, or less where the launch
+// would then leave CUs without a workgroup (ms per step, FP32 Poisson, single
+// phase / multiphase: 32^3 0.041 / 0.061 at 4 planes -> 0.036 / 0.047 at 1,
+// 64^3 0.046 / 0.068 -> 0.042 / 0.059 at 2).
+static int pass_chunk(const mhit_ctx* c, int mz, int my, int nb) {
+    const int n = c->n, zc = n < mz ? n : mz;
+    const long long tiles = (long long)div_up(n, tile_cols(my)) * div_up(n, my) * nb;
+    return tiles * div_up(n, zc) < c->cus ? chunk_planes(n, tiles, c->cus, zc) : zc;
+}
+
 template <typename TD>
-static NsArgs<TD> ns_args(mhit_ctx* c, TD* div) {
+static NsArgs<TD> ns_args(mhit_ctx* c, TD* div, int nb) {
     NsArgs<TD> a;
     a.u = c->u; a.v = c->v; a.w = c->w;
     a.phi = c->P.phiflag ? c->phi : nullptr;
@@ -565,12 +587,12 @@ static NsArgs<TD> ns_args(mhit_ctx* c, TD* div) {
     a.mysin = c->mysin; a.mycos = c->mycos;
     a.g = c->g;
     a.S = c->S;
-    a.zc = c->n < c->tune.ns_mz ? c->n : c->tune.ns_mz;
+    a.zc = pass_chunk(c, c->tune.ns_mz, c->tune.ns_my, nb);
     a.xcd = c->tune.xcd;
     return a;
 }
 
-static AcdiArgs acdi_args(mhit_ctx* c) {
+static AcdiArgs acdi_args(mhit_ctx* c, int nb) {
     AcdiArgs a;
     a.phi_out = c->phi_next;
     a.phi = c->phi;
@@ -578,7 +600,7 @@ static AcdiArgs acdi_args(mhit_ctx* c) {
     a.rphi_o = c->rhsphi_o;
     a.g = c->g;
     a.S = c->S;
-    a.zc = c->n < c->tune.ac_mz ? c->n : c->tune.ac_mz;
+    a.zc = pass_chunk(c, c->tune.ac_mz, c->tune.ac_my, nb);
     a.xcd = c->tune.xcd;
     return a;
 }
@@ -611,11 +633,11 @@ static void go_ns(mhit_ctx* c, const NsArgs<TD>& one, const NsArgs<TD>* tab, int
 // and the x C2R pass overwrites with p.
 int launch_ns_march(mhit_ctx* c) {
     if (c->P.phiflag) {
-        if (c->fp32) go_ns<true>(c, ns_args(c, (float*)c->pres), (const NsArgs<float>*)nullptr, 1, c->stream);
-        else go_ns<true>(c, ns_args(c, (double*)c->pres), (const NsArgs<double>*)nullptr, 1, c->stream);
+        if (c->fp32) go_ns<true>(c, ns_args(c, (float*)c->pres, 1), (const NsArgs<float>*)nullptr, 1, c->stream);
+        else go_ns<true>(c, ns_args(c, (double*)c->pres, 1), (const NsArgs<double>*)nullptr, 1, c->stream);
     } else {
-        if (c->fp32) go_ns<false>(c, ns_args(c, (float*)c->pres), (const NsArgs<float>*)nullptr, 1, c->stream);
-        else go_ns<false>(c, ns_args(c, (double*)c->pres), (const NsArgs<double>*)nullptr, 1, c->stream);
+        if (c->fp32) go_ns<false>(c, ns_args(c, (float*)c->pres, 1), (const NsArgs<float>*)nullptr, 1, c->stream);
+        else go_ns<false>(c, ns_args(c, (double*)c->pres, 1), (const NsArgs<double>*)nullptr, 1, c->stream);
     }
     prof_mark(c, ST_NS);
     MHIT_HIP_TRY(hipGetLastError());
@@ -626,7 +648,7 @@ int launch_ns_march(mhit_ctx* c) {
 template <bool PH, typename TD>
 static int ns_batch(mhit_ctx* const* boxes, int nb, ArgArena& arena, hipStream_t st) {
     std::vector<NsArgs<TD>> t(nb);
-    for (int b = 0; b < nb; b++) t[b] = ns_args(boxes[b], (TD*)boxes[b]->pres);
+    for (int b = 0; b < nb; b++) t[b] = ns_args(boxes[b], (TD*)boxes[b]->pres, nb);
     const NsArgs<TD>* tab = arena.put(t.data(), nb);
     if (!tab) { set_error("batched launch: argument arena full"); return MHIT_ERR_STATE; }
     go_ns<PH, TD>(boxes[0], t[0], tab, nb, st);
@@ -664,7 +686,7 @@ static void go_acdi(mhit_ctx* c, const AcdiArgs& one, const AcdiArgs* tab, int n
 }
 
 int launch_acdi_march(mhit_ctx* c) {
-    go_acdi(c, acdi_args(c), nullptr, 1, c->stream);
+    go_acdi(c, acdi_args(c, 1), nullptr, 1, c->stream);
     prof_mark(c, ST_ACDI);
     MHIT_HIP_TRY(hipGetLastError());
     std::swap(c->phi, c->phi_next);
@@ -680,7 +702,7 @@ int launch_acdi_march_batch(mhit_ctx* const* boxes, int nb, ArgArena& arena, hip
             set_error("batched ACDI pass: boxes differ in size or launch shape, or have no phase field");
             return MHIT_ERR_ARG;
         }
-        t[b] = acdi_args(boxes[b]);
+        t[b] = acdi_args(boxes[b], nb);
     }
     const AcdiArgs* tab = arena.put(t.data(), nb);
     if (!tab) { set_error("batched launch: argument arena full"); return MHIT_ERR_STATE; }

@@ -246,11 +246,10 @@ int mhit_autotune(mhit_ctx* c, int steps, mhit_tuning* out) {
     if ((rc = take(c, snap))) return rc;
 
     const int n = c->n;
-    auto zlist = [&](std::initializer_list<int> vals) {
-        std::vector<int> v;
+    auto zlist = [&](std::initializer_list<int> vals, int start) {
+        std::vector<int> v = {start};
         for (int z : vals)
-            if (z <= n) v.push_back(z);
-        if (v.empty()) v.push_back(n);
+            if (z <= n && z != start) v.push_back(z);
         return v;
     };
     auto widths = [&](int pass) {
@@ -261,9 +260,9 @@ int mhit_autotune(mhit_ctx* c, int steps, mhit_tuning* out) {
     struct Param { int* field; std::vector<int> cand; bool active; };
     std::vector<Param> params = {
         {&c->tune.ns_my, {16, 8, 32, 10}, true},
-        {&c->tune.ns_mz, zlist({4, 8, 16, 32, 64, 128}), true},
+        {&c->tune.ns_mz, zlist({4, 8, 16, 32, 64, 128}, c->tune.ns_mz), true},
         {&c->tune.ac_my, {16, 8, 32, 10}, c->P.phiflag != 0},
-        {&c->tune.ac_mz, zlist({4, 8, 16, 32, 64, 128}), c->P.phiflag != 0},
+        {&c->tune.ac_mz, zlist({4, 8, 16, 32, 64, 128}, c->tune.ac_mz), c->P.phiflag != 0},
         {&c->tune.xcd, {0, 1}, true},
         {&c->tune.fft_wave, {1, 0}, true},
         {&c->tune.fft_ycols, widths(0), widths(0).size() > 1},
