@@ -237,34 +237,42 @@ int launch_ns(mhit_ctx* c) {
 // ----------------------------------------------------------- correction
 // C, main.f90:942-962: u = u* - dt/rho (p - p(-1)) dxi with the pressure
 // promoted to FP64, plus per-block sums and maxima of the corrected u,v,w.
-// A workgroup owns a 64 x 8 (or 32 x 16) tile of columns and marches a chunk of z
-// planes (correct_zc): p(z-1) of its column stays in a register, the
-// plane's p with a one-point halo at -x and -y is staged in LDS, and the
-// next plane is fetched into registers during the update.  The number of partials is
-// fixed by the grid, so the reduction order is deterministic.
+// Bound by HBM: 52 (FP32 p) or 56 bytes per cell.
+//
+// Summation order.  The mean enters every velocity of the next step.  With
+// the FP32 Poisson a last-bit change of it flips roundings of div u* and so
+// replaces the whole FP32 rounding noise of p by another sample (2.5e-7 of
+// p, 1e-9 of u after ten steps at 256^3).  Its order is therefore fixed by
+// the grid size alone: 64 x 8 tiles (32 x 16 where n is a multiple of 32 but
+// not of 64: 96^3), chunks of correct_zc planes summed from the bottom up,
+// partials by 1024 interleaved runs.  With the FP64 Poisson the order is
+// fixed by the grid size too, but free to follow the faster sweep.
+//
+// k_correct takes a few planes of loads in flight per thread and p's
+// neighbours through the caches, without LDS and barriers.  In a running
+// step, march -> k_correct: 64^3 8.6 -> 7.0 us, 128^3 FP32 38 -> 24 us (4.5
+// TB/s), 192^3 FP64 102 -> 70 us (5.7 TB/s).  With the FP64 Poisson from
+// 256^3 its workgroups take 128 x 4 columns of two planes, so that the
+// dispatch order sweeps memory front to back: 512^3 1.36 -> 1.18 ms (6.3
+// TB/s); in the FP32 order's 16 and 32 planes per chunk it measured no
+// faster than the march there (512^3 1.24 - 1.29 against 1.24 ms, 256^3 157
+// against 156 us), which is kept for those.
 constexpr int CO_NT = 512;                    // threads per workgroup
-// tile columns: 64, or 32 where n is not a multiple of 64 (96^3: a
-// 64-column tile would leave a third of the threads without a cell); rows
-// make up the workgroup
-static int co_mx(int n) { return (n > 64 && n % 64 != 0 && n % 32 == 0) ? 32 : 64; }
-// z planes per workgroup: the longest of 32, 16, ..., 2 that gives a box
-// at least 256 workgroups (256^3: 32, 128^3: 16, 96^3: 8, 64^3 and below:
-// 2; at 64^3 8-plane chunks left 192 CUs idle, 14.8 us), and 16 from
-// 512^3 (1.36 -> 1.31 ms; 8 planes gain no more once the larger finalize
-// is counted; at 256^3 16 and 8 planes measured the same as 32).  A
-// function of n only, never of the device: the number of partials, and so
-// the reduction order, is fixed per grid size.
-static int correct_zc(int n) {
-    if (n >= 512) return 16;
-    const long long tiles = (long long)div_up(n, co_mx(n)) * div_up(n, CO_NT / co_mx(n));
-    int zc = 32;
-    while (zc > 2 && tiles * div_up(n, zc) < 256) zc /= 2;
-    return zc;
+struct CorrShape { int mx, my, zc; bool march; };
+static CorrShape correct_shape(int n, bool fp32) {
+    if (!fp32 && n >= 64) return {n >= 256 ? 128 : (n % 64 == 0 ? 64 : 32), n % 64 == 0 ? 4 : 16,
+                                  n >= 256 ? 2 : 4, false};
+    const int mx = (n > 64 && n % 64 != 0 && n % 32 == 0) ? 32 : 64, my = CO_NT / mx;
+    // the longest of 32, 16, ... 2 planes with at least 256 workgroups
+    const long long tiles = (long long)div_up(n, mx) * div_up(n, my);
+    int zc = n >= 512 ? 16 : 32;
+    while (n < 512 && zc > 2 && tiles * div_up(n, zc) < 256) zc /= 2;
+    return {mx, my, zc < n ? zc : n, n >= 256};
 }
 
-static dim3 correct_grid(int n) {
-    const int zc = correct_zc(n) < n ? correct_zc(n) : n;
-    return dim3(div_up(n, co_mx(n)), div_up(n, CO_NT / co_mx(n)), div_up(n, zc));
+static dim3 correct_grid(int n, bool fp32) {
+    const CorrShape s = correct_shape(n, fp32);
+    return dim3(div_up(n, s.mx), div_up(n, s.my), div_up(n, s.zc));
 }
 
 // Arguments of one box (a batched launch reads a table of them).
@@ -278,9 +286,88 @@ struct CorrArgs {
     int zc, xcd;
 };
 
+template <typename T, int MX, int MY, int U>
+__global__ __launch_bounds__(MX * MY)
+void k_correct(CorrArgs<T> one, const CorrArgs<T>* __restrict__ tab, int nbox) {
+    const Blk blk = launch_blk(nbox);
+    CorrArgs<T> A = one;
+    if (tab) A = tab[blk.box];
+    const MHIT_GLOBAL double* __restrict__ us = gmem(A.us);
+    const MHIT_GLOBAL double* __restrict__ vs = gmem(A.vs);
+    const MHIT_GLOBAL double* __restrict__ ws = gmem(A.ws);
+    const MHIT_GLOBAL T* __restrict__ p = gmem(A.p);
+    MHIT_GLOBAL double* __restrict__ u = gmem(A.u);
+    MHIT_GLOBAL double* __restrict__ v = gmem(A.v);
+    MHIT_GLOBAL double* __restrict__ w = gmem(A.w);
+    MHIT_GLOBAL double* __restrict__ partials = gmem(A.partials);
+    const Grid g = A.g;
+    const MHIT_GLOBAL DevScalars* __restrict__ S = gmem(A.S);
+    constexpr int NT = MX * MY;          // U planes in flight
+    __shared__ double red[6][NT / 64];
+    if (S->halted) return;               // the finalize pass reads no partials then
+    const int n = g.n;
+    const int tid = threadIdx.y * MX + threadIdx.x;
+    int tbx, tby, tbz;
+    xcd_tile(tbx, tby, tbz, blk, A.xcd);
+    const int i = tbx * MX + threadIdx.x, j = tby * MY + threadIdx.y;
+    const int z0 = tbz * A.zc, z1 = min(z0 + A.zc, n);
+    const double dtr = g.dt / g.rho;
+    double su = 0.0, sv = 0.0, sw = 0.0;
+    double mu_ = -INFINITY, mv_ = -INFINITY, mw_ = -INFINITY;
+    if (i < n && j < n) {
+        // in-plane offsets of the cell and of its -x and -y neighbours
+        const int o = j * n + i, ox = j * n + wrap_m(i, n), oy = wrap_m(j, n) * n + i;
+        const size_t plane = (size_t)n * n;
+        T pm = p[wrap_m(z0, n) * plane + o];
+        for (int k = z0; k < z1; k += U) {
+            T pc[U], px[U], py[U];
+            double uq[U], vq[U], wq[U];
+#pragma unroll
+            for (int t = 0; t < U; t++) {
+                if (k + t >= z1) continue;
+                const size_t b = (k + t) * plane;
+                pc[t] = p[b + o]; px[t] = p[b + ox]; py[t] = p[b + oy];
+                uq[t] = ld_once(&us[b + o]); vq[t] = ld_once(&vs[b + o]); wq[t] = ld_once(&ws[b + o]);
+            }
+#pragma unroll
+            for (int t = 0; t < U; t++) {
+                if (k + t >= z1) continue;
+                const size_t q = (k + t) * plane + o;
+                const double c = (double)pc[t];
+                const double uu = uq[t] - dtr * (c - (double)px[t]) * g.dxi;
+                const double vv = vq[t] - dtr * (c - (double)py[t]) * g.dxi;
+                const double ww = wq[t] - dtr * (c - (double)pm) * g.dxi;
+                st_once(&u[q], uu); st_once(&v[q], vv); st_once(&w[q], ww);
+                su += uu; sv += vv; sw += ww;
+                mu_ = fmax(mu_, uu); mv_ = fmax(mv_, vv); mw_ = fmax(mw_, ww);
+                pm = pc[t];
+            }
+        }
+    }
+    su = wave_sum(su); sv = wave_sum(sv); sw = wave_sum(sw);
+    mu_ = wave_max(mu_); mv_ = wave_max(mv_); mw_ = wave_max(mw_);
+    const int wv = tid >> 6;
+    if ((tid & 63) == 0) {
+        red[0][wv] = su; red[1][wv] = sv; red[2][wv] = sw;
+        red[3][wv] = mu_; red[4][wv] = mv_; red[5][wv] = mw_;
+    }
+    __syncthreads();
+    if (tid < 6) {
+        const int f = tid;
+        double r = red[f][0];
+        for (int t = 1; t < NT / 64; t++) r = (f < 3) ? r + red[f][t] : fmax(r, red[f][t]);
+        // partials in tile order, so the reduction order does not depend on
+        // the workgroup order (xcd_tile)
+        const size_t b = ((size_t)tbz * blk.ny + tby) * blk.nx + tbx;
+        partials[b * 6 + f] = r;
+    }
+}
+
+// The same with the column marched one plane at a time, p(z-1) of the column
+// in a register and the plane's p with a one-point halo at -x and -y in LDS.
 template <typename T, int CMX>
 __global__ __launch_bounds__(CO_NT)
-void k_correct(CorrArgs<T> one, const CorrArgs<T>* __restrict__ tab, int nbox) {
+void k_correct_march(CorrArgs<T> one, const CorrArgs<T>* __restrict__ tab, int nbox) {
     const Blk blk = launch_blk(nbox);
     CorrArgs<T> A = one;
     if (tab) A = tab[blk.box];
@@ -386,20 +473,40 @@ static CorrArgs<T> corr_args(mhit_ctx* c) {
     a.partials = c->partials;
     a.g = c->g;
     a.S = c->S;
-    a.zc = correct_zc(c->n) < c->n ? correct_zc(c->n) : c->n;
-    // XCD-aware tile order always: neighbouring tiles' p halo rows then hit
-    // in the same L2 (1.39 -> 1.36 ms at 512^3; the partials are indexed by
-    // tile, so the order changes no bit)
-    a.xcd = 1;
+    const CorrShape sh = correct_shape(c->n, c->fp32);
+    a.zc = sh.zc;
+    // XCD tile order where p's neighbours then hit in the same L2: the march
+    // (1.39 -> 1.36 ms at 512^3) and small boxes (96^3 10.9 against 11.3 us);
+    // the partials are indexed by tile, so the order changes no bit
+    a.xcd = sh.march || c->n < 192;
     return a;
 }
 
 template <typename T>
 static void go_correct(int n, const CorrArgs<T>& one, const CorrArgs<T>* tab, int nb, hipStream_t st) {
-    dim3 grid = correct_grid(n);
+    constexpr bool F32 = sizeof(T) == 4;
+    const CorrShape sh = correct_shape(n, F32);
+    dim3 grid = correct_grid(n, F32);
     grid.z *= nb;
-    if (co_mx(n) == 32) k_correct<T, 32><<<grid, dim3(32, CO_NT / 32, 1), 0, st>>>(one, tab, nb);
-    else k_correct<T, 64><<<grid, dim3(64, CO_NT / 64, 1), 0, st>>>(one, tab, nb);
+    const dim3 block(sh.mx, sh.my, 1);
+    if constexpr (F32) {
+        if (sh.march) {
+            k_correct_march<T, 64><<<grid, block, 0, st>>>(one, tab, nb);
+            return;
+        }
+    } else {
+        if (sh.mx == 128) {
+            k_correct<T, 128, 4, 2><<<grid, block, 0, st>>>(one, tab, nb);
+            return;
+        }
+        if (sh.my == 4) {
+            k_correct<T, 64, 4, 2><<<grid, block, 0, st>>>(one, tab, nb);
+            return;
+        }
+    }
+    if (sh.mx == 32) k_correct<T, 32, 16, 2><<<grid, block, 0, st>>>(one, tab, nb);
+    else if (n >= 192) k_correct<T, 64, 8, 4><<<grid, block, 0, st>>>(one, tab, nb);
+    else k_correct<T, 64, 8, 2><<<grid, block, 0, st>>>(one, tab, nb);
 }
 
 int launch_correct(mhit_ctx* c) {
@@ -431,11 +538,145 @@ int launch_correct_batch(mhit_ctx* const* boxes, int nb, ArgArena& arena, hipStr
     return c->fp32 ? correct_batch<float>(boxes, nb, arena, st) : correct_batch<double>(boxes, nb, arena, st);
 }
 
-int correct_block_count(int n) {
-    const dim3 g = correct_grid(n);
+// Finalize: means (main.f90:964-974), signed max after the mean removal
+// (998-1002, max(u - m) = max(u) - m as rounding is monotone), CFL
+// (1003-1006), AB2 switch (801-802).  One workgroup, fixed reduction order:
+// thread t adds up partials t, t + 1024, ..., then a tree over the threads.
+// Above kFinMost partials (the FP64 sweeps of large boxes) k_fin_parts first
+// adds up runs of kFinPart of them.
+constexpr int kFinMost = 4096, kFinPart = 64;
+
+static int fin_parts(int n, bool fp32) {
+    const int nb = correct_block_count(n, fp32);
+    return !fp32 && nb > kFinMost ? div_up(nb, kFinPart) : 0;
+}
+int correct_block_count(int n, bool fp32) {
+    const dim3 g = correct_grid(n, fp32);
     return (int)(g.x * g.y * g.z);
 }
+// space for the partials, in doubles: the correction's, then their sums
+size_t correct_partials(int n, bool fp32) {
+    return (size_t)(correct_block_count(n, fp32) + fin_parts(n, fp32)) * 6;
+}
 
+struct FinArgs {
+    double* partials;
+    int nblocks, nparts, cfl_abort;   // partials, and sums of runs of them (0: none)
+    Grid g;
+    DevScalars* S;
+};
+
+// A wave per run of kFinPart partials; blockIdx.y is the box of a batched
+// launch.
+__global__ __launch_bounds__(256)
+void k_fin_parts(FinArgs one, const FinArgs* __restrict__ tab) {
+    FinArgs A = one;
+    if (tab) A = tab[blockIdx.y];
+    if (gmem(A.S)->halted) return;
+    const int run = blockIdx.x * 4 + (threadIdx.x >> 6), b = run * kFinPart + (threadIdx.x & 63);
+    if (run >= A.nparts) return;
+    MHIT_GLOBAL double* partials = gmem(A.partials);
+    const bool on = b < A.nblocks;
+    for (int f = 0; f < 6; f++) {
+        const double x = on ? partials[(size_t)b * 6 + f] : (f < 3 ? 0.0 : -INFINITY);
+        const double r = f < 3 ? wave_sum(x) : wave_max(x);
+        if ((threadIdx.x & 63) == 0) partials[(size_t)(A.nblocks + run) * 6 + f] = r;
+    }
+}
+
+// One workgroup per box (blockIdx.x is the box of a batched launch).
+__global__ __launch_bounds__(1024)
+void k_finalize(FinArgs one, const FinArgs* __restrict__ tab) {
+    FinArgs A = one;
+    if (tab) A = tab[blockIdx.x];
+    const Grid g = A.g;
+    MHIT_GLOBAL DevScalars* __restrict__ S = gmem(A.S);
+    const MHIT_GLOBAL double* __restrict__ partials = gmem(A.partials) + (A.nparts ? (size_t)A.nblocks * 6 : 0);
+    const int nblocks = A.nparts ? A.nparts : A.nblocks;
+    __shared__ double red[6][512];
+    const int t = threadIdx.x;
+    if (S->halted) {
+        if (t == 0) S->skipped += 1;   // a step whose passes all returned at once
+        return;
+    }
+    double a[6] = {0.0, 0.0, 0.0, -INFINITY, -INFINITY, -INFINITY};
+    for (int b = t; b < nblocks; b += 1024) {
+        for (int f = 0; f < 3; f++) a[f] += partials[(size_t)b * 6 + f];
+        for (int f = 3; f < 6; f++) a[f] = fmax(a[f], partials[(size_t)b * 6 + f]);
+    }
+    // thread t takes up t + 512, t + 256, ..., t + 1: the first four through
+    // LDS, the rest within the wave
+    for (int s = 512; s >= 64; s >>= 1) {
+        if (t >= s && t < 2 * s)
+            for (int f = 0; f < 6; f++) red[f][t - s] = a[f];
+        __syncthreads();
+        if (t < s)
+            for (int f = 0; f < 6; f++) a[f] = f < 3 ? a[f] + red[f][t] : fmax(a[f], red[f][t]);
+        __syncthreads();
+    }
+    if (t >= 64) return;
+    for (int s = 32; s > 0; s >>= 1)
+        for (int f = 0; f < 6; f++) {
+            const double x = __shfl_down(a[f], s, 64);
+            a[f] = f < 3 ? a[f] + x : fmax(a[f], x);
+        }
+    if (t == 0) {
+        const double nn = (double)g.n;
+        double m[3], mx[3];
+        for (int f = 0; f < 3; f++) {
+            m[f] = a[f] / nn / nn / nn;
+            mx[f] = a[f + 3] - m[f];
+        }
+        const double umax = fmax(mx[2], fmax(mx[0], mx[1]));
+        S->mean[0] = m[0]; S->mean[1] = m[1]; S->mean[2] = m[2];
+        S->gumax = umax;
+        S->cou = umax * g.dt * g.dxi;
+        S->alpha = 1.5;
+        S->beta = 0.5;
+        S->step += 1;
+        if (A.cfl_abort && S->cou > 7.0) S->halted = 1;
+    }
+}
+
+static FinArgs fin_args(mhit_ctx* c) {
+    FinArgs a;
+    a.partials = c->partials;
+    a.nblocks = c->npart_blocks;
+    a.nparts = fin_parts(c->n, c->fp32);
+    a.cfl_abort = c->P.cfl_abort;
+    a.g = c->g;
+    a.S = c->S;
+    return a;
+}
+
+static void go_finalize(const FinArgs& one, const FinArgs* tab, int nb, int nparts, hipStream_t st) {
+    if (nparts) k_fin_parts<<<dim3(div_up(nparts, 4), nb), 256, 0, st>>>(one, tab);
+    k_finalize<<<nb, 1024, 0, st>>>(one, tab);
+}
+
+int launch_finalize(mhit_ctx* c) {
+    const FinArgs a = fin_args(c);
+    go_finalize(a, nullptr, 1, a.nparts, c->stream);
+    prof_mark(c, ST_FINALIZE);
+    MHIT_HIP_TRY(hipGetLastError());
+    return MHIT_OK;
+}
+
+int launch_finalize_batch(mhit_ctx* const* boxes, int nb, ArgArena& arena, hipStream_t st) {
+    std::vector<FinArgs> t(nb);
+    int nparts = 0;
+    for (int b = 0; b < nb; b++) {
+        t[b] = fin_args(boxes[b]);
+        nparts = std::max(nparts, t[b].nparts);
+    }
+    const FinArgs* tab = arena.put(t.data(), nb);
+    if (!tab) { set_error("batched launch: argument arena full"); return MHIT_ERR_STATE; }
+    go_finalize(t[0], tab, nb, nparts, st);
+    MHIT_HIP_TRY(hipGetLastError());
+    return MHIT_OK;
+}
+
+// ---------------------------------------------------------- diagnostics
 // Diagnostics: 64 x 8 columns per workgroup, chunks of 32 planes from
 // 512^3, 16 from 256^3 and 4 below (each chunk reads two planes more; short
 // chunks keep small boxes on all CUs).
@@ -447,91 +688,6 @@ int diag_block_count(int n) {
     return (int)(g.x * g.y * g.z);
 }
 
-// Finalize: means (main.f90:964-974), signed max after the mean removal
-// (998-1002, max(u - m) = max(u) - m as rounding is monotone), CFL
-// (1003-1006), AB2 switch (801-802).  One block, fixed reduction order.
-struct FinArgs {
-    const double* partials;
-    int nblocks, cfl_abort;
-    Grid g;
-    DevScalars* S;
-};
-
-// One workgroup per box (blockIdx.x is the box of a batched launch).
-__global__ __launch_bounds__(1024)
-void k_finalize(FinArgs one, const FinArgs* __restrict__ tab) {
-    FinArgs A = one;
-    if (tab) A = tab[blockIdx.x];
-    const MHIT_GLOBAL double* __restrict__ partials = gmem(A.partials);
-    const int nblocks = A.nblocks, cfl_abort = A.cfl_abort;
-    const Grid g = A.g;
-    MHIT_GLOBAL DevScalars* __restrict__ S = gmem(A.S);
-    __shared__ double red[6][1024];
-    const int t = threadIdx.x;
-    if (S->halted) {
-        if (t == 0) S->skipped += 1;   // a step whose passes all returned at once
-        return;
-    }
-    double a[6] = {0.0, 0.0, 0.0, -INFINITY, -INFINITY, -INFINITY};
-    for (int b = t; b < nblocks; b += 1024) {
-        for (int f = 0; f < 3; f++) a[f] += partials[(size_t)b * 6 + f];
-        for (int f = 3; f < 6; f++) a[f] = fmax(a[f], partials[(size_t)b * 6 + f]);
-    }
-    for (int f = 0; f < 6; f++) red[f][t] = a[f];
-    __syncthreads();
-    for (int s = 512; s > 0; s >>= 1) {
-        if (t < s) {
-            for (int f = 0; f < 3; f++) red[f][t] += red[f][t + s];
-            for (int f = 3; f < 6; f++) red[f][t] = fmax(red[f][t], red[f][t + s]);
-        }
-        __syncthreads();
-    }
-    if (t == 0) {
-        const double nn = (double)g.n;
-        double m[3], mx[3];
-        for (int f = 0; f < 3; f++) {
-            m[f] = red[f][0] / nn / nn / nn;
-            mx[f] = red[f + 3][0] - m[f];
-        }
-        const double umax = fmax(mx[2], fmax(mx[0], mx[1]));
-        S->mean[0] = m[0]; S->mean[1] = m[1]; S->mean[2] = m[2];
-        S->gumax = umax;
-        S->cou = umax * g.dt * g.dxi;
-        S->alpha = 1.5;
-        S->beta = 0.5;
-        S->step += 1;
-        if (cfl_abort && S->cou > 7.0) S->halted = 1;
-    }
-}
-
-static FinArgs fin_args(mhit_ctx* c) {
-    FinArgs a;
-    a.partials = c->partials;
-    a.nblocks = c->npart_blocks;
-    a.cfl_abort = c->P.cfl_abort;
-    a.g = c->g;
-    a.S = c->S;
-    return a;
-}
-
-int launch_finalize(mhit_ctx* c) {
-    k_finalize<<<1, 1024, 0, c->stream>>>(fin_args(c), nullptr);
-    prof_mark(c, ST_FINALIZE);
-    MHIT_HIP_TRY(hipGetLastError());
-    return MHIT_OK;
-}
-
-int launch_finalize_batch(mhit_ctx* const* boxes, int nb, ArgArena& arena, hipStream_t st) {
-    std::vector<FinArgs> t(nb);
-    for (int b = 0; b < nb; b++) t[b] = fin_args(boxes[b]);
-    const FinArgs* tab = arena.put(t.data(), nb);
-    if (!tab) { set_error("batched launch: argument arena full"); return MHIT_ERR_STATE; }
-    k_finalize<<<nb, 1024, 0, st>>>(t[0], tab);
-    MHIT_HIP_TRY(hipGetLastError());
-    return MHIT_OK;
-}
-
-// ---------------------------------------------------------- diagnostics
 // KE, dissipation 2 nu <S_ij S_ij> with central differences
 // (post/compute_diss/main.f90:72-117, dx = lx/n, nu = mu/rho), max |D.u|
 // with the divergence stencil of main.f90:841-843, phi mass and range.

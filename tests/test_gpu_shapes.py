@@ -31,3 +31,26 @@ def test_default_shapes_against_others(n, prec, shape):
     print(f"[shapes] n={n} prec={prec} {shape}", flush=True)
     for f, (a, b) in enumerate(zip(_run(n, prec), _run(n, prec, **shape)), start=1):
         assert np.array_equal(a, b), f
+
+
+@pytest.mark.parametrize("prec", [0, 1], ids=["fp64", "fp32"])
+@pytest.mark.parametrize("n", [8, 12, 24, 48, 64, 96, 128, 192, 256])
+def test_correction_mean_and_max(n, prec):
+    """The means that a step removes and its signed maximum, over tiles that
+    overhang the grid, one and two levels of partial sums: the removed mean
+    is the initial one (every term of the step sums to zero over the box up
+    to rounding), the downloaded velocity has zero mean (sums of n^3 terms of
+    order one in FP64) and its maximum is the reported one to the last bit."""
+    from mhit36_mixedp_amd import Solver
+    print(f"[shapes] correction n={n} prec={prec}", flush=True)
+    rng = np.random.default_rng(n)
+    with Solver(nx=n, poisson_precision=prec, dt=1e-4, mu=0.01) as s:
+        start = [rng.standard_normal((n, n, n)) + m for m in (0.5, -0.25, 0.125)]
+        s.set_velocity(*start)
+        s.step(1)
+        vel = s.velocity()
+        d = s.scalars()
+        for v, v0, m in zip(vel, start, ("umean", "vmean", "wmean")):
+            assert abs(v.mean()) < 1e-13
+            assert abs(d[m] - v0.mean()) < 1e-12
+        assert d["gumax"] == max(v.max() for v in vel)
