@@ -15,6 +15,7 @@ from . import _abi
 from ._abi import Diag, Params, default_params
 
 _dp = ctypes.POINTER(ctypes.c_double)
+_DROP = np.dtype(_abi.Drop)   # mhit_drop, one record per drop
 
 
 class MhitError(RuntimeError):
@@ -223,13 +224,13 @@ class Solver:
     def drop_stats(self, threshold: float = 0.5, connectivity: int = 6, max_drops: int = 1 << 16):
         """Connected drops of phi >= threshold (see mhit_drop_stats); a dict of
         numpy columns, one entry per drop, ordered by first cell."""
-        buf = (_abi.Drop * max(1, max_drops))()
+        buf = np.zeros(max(1, max_drops), dtype=_DROP)
         nd = ctypes.c_int64()
         _check(self.lib.mhit_drop_stats(self._h, float(threshold), int(connectivity), int(max_drops),
-                                        buf, ctypes.byref(nd)), "mhit_drop_stats")
+                                        buf.ctypes.data_as(ctypes.POINTER(_abi.Drop)), ctypes.byref(nd)),
+               "mhit_drop_stats")
         k = min(nd.value, max_drops)
-        names = [f for f, _ in _abi.Drop._fields_]
-        out = {f: np.array([getattr(buf[i], f) for i in range(k)]) for f in names}
+        out = {f: buf[f][:k].copy() for f in _DROP.names}
         out["count"] = nd.value
         return out
 

@@ -58,7 +58,6 @@ struct mhit_ensemble {
     // the boxes' scalars read back in one copy: a device table of their
     // DevScalars pointers, a device gather buffer and its pinned host copy
     const DevScalars** s_src = nullptr;
-    DevScalars* s_dev = nullptr;
     DevScalars* s_host = nullptr;
 };
 
@@ -66,21 +65,22 @@ __global__ void k_gather_scalars(const DevScalars* const* __restrict__ src, DevS
                                  int nb) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b < nb) dst[b] = *src[b];
+    __threadfence_system();   // dst is pinned host memory
 }
 
 // After the replays on the ensemble stream: every box's scalars to the host
-// with one gather kernel and one copy (one round trip instead of one per
-// box), then each box's own end-of-call bookkeeping.
+// with one gather kernel that stores to pinned memory (one round trip instead
+// of one per box), then each box's own end-of-call bookkeeping.
 static int finish_ensemble(mhit_ensemble* e, int* status) {
     const int nb = (int)e->boxes.size();
-    k_gather_scalars<<<div_up(nb, 64), 64, 0, e->stream>>>(e->s_src, e->s_dev, nb);
+    k_gather_scalars<<<div_up(nb, 64), 64, 0, e->stream>>>(e->s_src, e->s_host, nb);
     MHIT_HIP_TRY(hipGetLastError());
-    MHIT_HIP_TRY(hipMemcpyAsync(e->s_host, e->s_dev, nb * sizeof(DevScalars), hipMemcpyDeviceToHost, e->stream));
     MHIT_HIP_TRY(hipStreamSynchronize(e->stream));
     *status = MHIT_OK;
     for (int b = 0; b < nb; b++) {
         mhit_ctx* c = e->boxes[b];
         c->S_host = e->s_host[b];
+        c->S_queued = false;
         const int rc = finish_synced(c);
         if (rc == MHIT_ERR_CFL) *status = MHIT_ERR_CFL;
         else if (rc) return rc;
@@ -332,6 +332,7 @@ static int ensemble_graph_step(mhit_ensemble* e) {
         if ((rc = can_batch(e) ? capture_ensemble_batched(e, slot) : capture_ensemble_step(e, slot)))
             return rc;
     }
+    for (mhit_ctx* c : e->boxes) c->S_queued = true;
     MHIT_HIP_TRY(hipGraphLaunch(slot->exec, e->stream));
     for (size_t b = 0; b < e->boxes.size(); b++)
         pingpong_apply(e->boxes[b], slot->box[b].in, slot->box[b].out);
@@ -364,7 +365,6 @@ int mhit_ensemble_create(int32_t nbox, const mhit_params* params, mhit_ensemble*
     std::vector<const DevScalars*> src(nbox);
     for (int32_t b = 0; b < nbox; b++) src[b] = e->boxes[b]->S;
     ok = ok && hipMalloc((void**)&e->s_src, nbox * sizeof(DevScalars*)) == hipSuccess &&
-         hipMalloc((void**)&e->s_dev, nbox * sizeof(DevScalars)) == hipSuccess &&
          hipHostMalloc((void**)&e->s_host, nbox * sizeof(DevScalars), hipHostMallocDefault) == hipSuccess &&
          hipMemcpy(e->s_src, src.data(), nbox * sizeof(DevScalars*), hipMemcpyHostToDevice) == hipSuccess;
     if (!ok) {
@@ -598,7 +598,6 @@ int mhit_ensemble_destroy(mhit_ensemble* e) {
     if (e->fork) (void)hipEventDestroy(e->fork);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     if (e->s_src) (void)hipFree(e->s_src);
-    if (e->s_dev) (void)hipFree(e->s_dev);
     if (e->s_host) (void)hipHostFree(e->s_host);
     delete e;
     return MHIT_OK;

@@ -68,6 +68,9 @@ struct mhit_ctx {
     double* drop_buf = nullptr;   // drop statistics: tables, list and sums (drops.hip)
     // host copy of scalars after the last sync
     mhit::DevScalars S_host{};
+    mhit::DevScalars* S_pin = nullptr;   // pinned: where the device puts them
+    double* diag_pin = nullptr;          // pinned: the diagnostics' eight sums, behind S_pin
+    bool S_queued = false;               // a step may have changed S since S_host was read
     // captured timesteps, keyed by the buffers they use (phi ping-pong
     // parity, tracer columns after a re-ordering)
     // buffer pairs whose roles alternate from step to step

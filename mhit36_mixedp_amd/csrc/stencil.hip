@@ -787,6 +787,7 @@ void k_diag_sum(const double* __restrict__ partials, int nb, double* __restrict_
     if (t == 0) {
         for (int v = 1; v < 16; v++) r = diag_join(f, r, red[v]);
         out[f] = r;
+        __threadfence_system();   // out is pinned host memory
     }
 }
 
@@ -841,12 +842,12 @@ int launch_stream_probe(mhit_ctx* c, const double* const* in, int R, double* con
 
 int launch_diag(mhit_ctx* c, double* out) {
     const int nb = c->ndiag_blocks;
-    double* sum = c->dpartials + (size_t)nb * NF;
     k_diag<<<diag_grid(c->n), dim3(64, DI_MY, 1), 0, c->stream>>>(
         c->u, c->v, c->w, c->P.phiflag ? c->phi : nullptr, c->dpartials, c->g, diag_zc(c->n), c->S);
-    k_diag_sum<<<NF, 1024, 0, c->stream>>>(c->dpartials, nb, sum);
+    k_diag_sum<<<NF, 1024, 0, c->stream>>>(c->dpartials, nb, c->diag_pin);
     MHIT_HIP_TRY(hipGetLastError());
-    MHIT_HIP_TRY(copy_on_stream(c, out, sum, NF * sizeof(double), hipMemcpyDeviceToHost));
+    MHIT_HIP_TRY(hipStreamSynchronize(c->stream));
+    for (int f = 0; f < NF; f++) out[f] = c->diag_pin[f];
     return MHIT_OK;
 }
 
