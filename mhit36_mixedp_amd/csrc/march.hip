@@ -23,10 +23,15 @@
 
 namespace mhit {
 
+// periodic index of a >= -n (a tile overhangs the grid by less than a tile,
+// so the loop ends at once unless the grid is smaller than the tile)
 __device__ __forceinline__ int wrapn(int a, int n) {
-    a %= n;
-    return a < 0 ? a + n : a;
+    if (a < 0) a += n;
+    while (a >= n) a -= n;
+    return a;
 }
+// periodic plane index of -n <= k < 2 n
+__device__ __forceinline__ int wrapk(int k, int n) { return k < 0 ? k + n : (k >= n ? k - n : k); }
 __device__ __forceinline__ int ring3(int k) { return ((k % 3) + 3) % 3; }
 __device__ __forceinline__ int ring4(int k) { return ((k % 4) + 4) % 4; }
 
@@ -109,12 +114,13 @@ void k_ns_march(NsArgs<TD> one, const NsArgs<TD>* __restrict__ tab, int nbox) {
     const int z0 = tbz * zc;
     const int z1 = min(z0 + zc, n);
     const int i = i0 + tx, j = j0 + ty;
-    const bool live = i < n && j < n;
     // A stopped run writes nothing; its AB2 history stays in the buffer it
     // was in, and the host undoes an odd number of buffer swaps afterwards
-    // (the finalize pass counts the skipped steps).  No copy here: any code
-    // in this branch costs the marching loop registers.
-    if (S->halted) return;
+    // (the finalize pass counts the skipped steps).  The flag is looked at
+    // where something is stored, as in every pass of a step: returning on it
+    // first would put its load in front of all others (about 0.6 us of each
+    // launch).
+    const bool live = i < n && j < n && !S->halted;
     // global indices of the cell, or of its periodic image past the domain edge
     const int ic = wrapn(i, n), jc = wrapn(j, n);
     const double m0 = S->mean[0], m1 = S->mean[1], m2 = S->mean[2];
@@ -143,7 +149,7 @@ void k_ns_march(NsArgs<TD> one, const NsArgs<TD>* __restrict__ tab, int nbox) {
     }
     struct Plane { double u[NV], v[NV], w[NV], p[PHI ? NPH : 1]; };
     auto fetch = [&](int k, Plane& r) {
-        const size_t base = (size_t)wrapn(k, n) * plane;
+        const size_t base = (size_t)wrapk(k, n) * plane;
 #pragma unroll
         for (int t = 0; t < NV; t++) {
             if ((H1 * W1) % NT == 0 || tid + t * NT < H1 * W1) {
@@ -265,7 +271,7 @@ void k_ns_march(NsArgs<TD> one, const NsArgs<TD>* __restrict__ tab, int nbox) {
     double dprev = 0.0, wsprev = 0.0;   // divergence partial and w* of the previous plane
     for (int k = z0; k <= z1; k++) {
         const bool last = k == z1;      // one plane past the chunk: w* only
-        const int kg = last ? wrapn(k, n) : k;
+        const int kg = last ? wrapk(k, n) : k;
         // AB2 history of the own column: issued before the barriers
         const size_t q = idx3(ic, jc, kg, n);
         const double row = rw_o[q];
@@ -387,13 +393,6 @@ void k_acdi_march(AcdiArgs one, const AcdiArgs* __restrict__ tab, int nbox) {
     const int z1 = min(z0 + zc, n);
     const int i = i0 + tx, j = j0 + ty;
     const bool live = i < n && j < n;
-    if (S->halted) {
-        // a stopped run keeps its state: phi_out becomes a copy of phi, so
-        // the host-side ping-pong of the two buffers stays consistent
-        if (live)
-            for (int k = z0; k < z1; k++) phi_out[idx3(i, j, k, n)] = phi[idx3(i, j, k, n)];
-        return;
-    }
     const double m0 = S->mean[0], m1 = S->mean[1], m2 = S->mean[2];
     const double alpha = S->alpha, beta = S->beta;
     const double gamma = 1.0 * S->gumax;               // main.f90:536
@@ -413,7 +412,7 @@ void k_acdi_march(AcdiArgs one, const AcdiArgs* __restrict__ tab, int nbox) {
     }
     struct Plane { double p[NPL]; };
     auto fetch = [&](int k, Plane& r) {
-        const MHIT_GLOBAL double* __restrict__ pl = phi + (size_t)wrapn(k, n) * plane;
+        const MHIT_GLOBAL double* __restrict__ pl = phi + (size_t)wrapk(k, n) * plane;
 #pragma unroll
         for (int t = 0; t < NPL; t++)
             if ((H2 * W2) % NT == 0 || tid + t * NT < H2 * W2) r.p[t] = pl[poff[t]];
@@ -498,6 +497,13 @@ void k_acdi_march(AcdiArgs one, const AcdiArgs* __restrict__ tab, int nbox) {
         fetch(z0, r0);
         fetch(z0 + 1, rp);
         fetch(z0 + 2, nx);
+        if (S->halted) {
+            // a stopped run keeps its state: phi_out becomes a copy of phi, so
+            // the host-side ping-pong of the two buffers stays consistent
+            if (live)
+                for (int k = z0; k < z1; k++) phi_out[idx3(i, j, k, n)] = phi[idx3(i, j, k, n)];
+            return;
+        }
         commit(z0 - 2, r2);
         commit(z0 - 1, r1);
         commit(z0, r0);

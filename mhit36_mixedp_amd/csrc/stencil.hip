@@ -304,13 +304,13 @@ void k_correct(CorrArgs<T> one, const CorrArgs<T>* __restrict__ tab, int nbox) {
     const MHIT_GLOBAL DevScalars* __restrict__ S = gmem(A.S);
     constexpr int NT = MX * MY;          // U planes in flight
     __shared__ double red[6][NT / 64];
-    if (S->halted) return;               // the finalize pass reads no partials then
     const int n = g.n;
     const int tid = threadIdx.y * MX + threadIdx.x;
     int tbx, tby, tbz;
     xcd_tile(tbx, tby, tbz, blk, A.xcd);
     const int i = tbx * MX + threadIdx.x, j = tby * MY + threadIdx.y;
     const int z0 = tbz * A.zc, z1 = min(z0 + A.zc, n);
+    const bool halted = S->halted;       // looked at before the stores
     const double dtr = g.dt / g.rho;
     double su = 0.0, sv = 0.0, sw = 0.0;
     double mu_ = -INFINITY, mv_ = -INFINITY, mw_ = -INFINITY;
@@ -337,7 +337,7 @@ void k_correct(CorrArgs<T> one, const CorrArgs<T>* __restrict__ tab, int nbox) {
                 const double uu = uq[t] - dtr * (c - (double)px[t]) * g.dxi;
                 const double vv = vq[t] - dtr * (c - (double)py[t]) * g.dxi;
                 const double ww = wq[t] - dtr * (c - (double)pm) * g.dxi;
-                st_once(&u[q], uu); st_once(&v[q], vv); st_once(&w[q], ww);
+                if (!halted) { st_once(&u[q], uu); st_once(&v[q], vv); st_once(&w[q], ww); }
                 su += uu; sv += vv; sw += ww;
                 mu_ = fmax(mu_, uu); mv_ = fmax(mv_, vv); mw_ = fmax(mw_, ww);
                 pm = pc[t];
@@ -595,10 +595,7 @@ void k_finalize(FinArgs one, const FinArgs* __restrict__ tab) {
     const int nblocks = A.nparts ? A.nparts : A.nblocks;
     __shared__ double red[6][512];
     const int t = threadIdx.x;
-    if (S->halted) {
-        if (t == 0) S->skipped += 1;   // a step whose passes all returned at once
-        return;
-    }
+    const bool halted = S->halted;     // partials of a stopped run are not used
     double a[6] = {0.0, 0.0, 0.0, -INFINITY, -INFINITY, -INFINITY};
     for (int b = t; b < nblocks; b += 1024) {
         for (int f = 0; f < 3; f++) a[f] += partials[(size_t)b * 6 + f];
@@ -620,7 +617,8 @@ void k_finalize(FinArgs one, const FinArgs* __restrict__ tab) {
             const double x = __shfl_down(a[f], s, 64);
             a[f] = f < 3 ? a[f] + x : fmax(a[f], x);
         }
-    if (t == 0) {
+    if (t == 0 && halted) S->skipped += 1;   // a step that stored nothing
+    if (t == 0 && !halted) {
         const double nn = (double)g.n;
         double m[3], mx[3];
         for (int f = 0; f < 3; f++) {
