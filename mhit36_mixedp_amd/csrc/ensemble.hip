@@ -185,7 +185,9 @@ static int enqueue_size_class(const std::vector<mhit_ctx*>& boxes, ArgArena& ar,
         if ((rc = poisson_project_batch(gp.data(), (int)gp.size(), ar, st))) return rc;
     for (auto& gp : by_prec)
         if ((rc = launch_correct_batch(gp.data(), (int)gp.size(), ar, st))) return rc;
-    return launch_finalize_batch(boxes.data(), (int)boxes.size(), ar, st);
+    for (auto& gp : by_prec)
+        if ((rc = launch_finalize_batch(gp.data(), (int)gp.size(), ar, st))) return rc;
+    return MHIT_OK;
 }
 
 // Launch shapes for boxes batched in an ensemble: 64 x 16 tiles (96 x 10

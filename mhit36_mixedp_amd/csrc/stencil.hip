@@ -249,16 +249,17 @@ int launch_ns(mhit_ctx* c) {
 // fixed by the grid size too, but free to follow the faster sweep.
 //
 // k_correct takes a few planes of loads in flight per thread and p's
-// neighbours through the caches, without LDS and barriers.  In a running
-// step, march -> k_correct: 64^3 8.6 -> 7.0 us, 128^3 FP32 38 -> 24 us (4.5
-// TB/s), 192^3 FP64 102 -> 70 us (5.7 TB/s).  With the FP64 Poisson from
-// 256^3 its workgroups take 128 x 4 columns of two planes, so that the
-// dispatch order sweeps memory front to back: 512^3 1.36 -> 1.18 ms (6.3
-// TB/s); in the FP32 order's 16 and 32 planes per chunk it measured no
-// faster than the march there (512^3 1.24 - 1.29 against 1.24 ms, 256^3 157
-// against 156 us), which is kept for those.
-constexpr int CO_NT = 512;                    // threads per workgroup
-struct CorrShape { int mx, my, zc; bool march; };
+// neighbours through the caches, without LDS and barriers.  (Marching one
+// plane at a time with p in LDS behind a barrier, in a running step: 64^3
+// 8.6 -> 7.0 us, 128^3 FP32 38 -> 24 us, 192^3 FP64 102 -> 70 us.)  From
+// 256^3 its workgroups are wide and flat, so that the dispatch order sweeps
+// memory front to back.  FP64: 128 x 4 columns of two planes, 512^3 1.36 ->
+// 1.18 ms (6.3 TB/s).  FP32: rows of 256 cells (128 x 2 where n is no
+// multiple of 256) over the order's chunk, 512^3 1.27 -> 1.22 ms, 384^3 0.59
+// -> 0.54, 256^3 0.172 -> 0.158 (5.5 TB/s) against the march; a wave writes
+// its row's sums and k_fin_rows (4 us) adds them up as an 8-row tile would.
+constexpr int CO_NT = 512;                    // threads per workgroup of the 8-row tile
+struct CorrShape { int mx, my, zc; bool rows; };
 static CorrShape correct_shape(int n, bool fp32) {
     if (!fp32 && n >= 64) return {n >= 256 ? 128 : (n % 64 == 0 ? 64 : 32), n % 64 == 0 ? 4 : 16,
                                   n >= 256 ? 2 : 4, false};
@@ -267,7 +268,8 @@ static CorrShape correct_shape(int n, bool fp32) {
     const long long tiles = (long long)div_up(n, mx) * div_up(n, my);
     int zc = n >= 512 ? 16 : 32;
     while (n < 512 && zc > 2 && tiles * div_up(n, zc) < 256) zc /= 2;
-    return {mx, my, zc < n ? zc : n, n >= 256};
+    if (n >= 256 && n % 128 == 0) return {n % 256 == 0 ? 256 : 128, n % 256 == 0 ? 1 : 2, zc, true};
+    return {mx, my, zc < n ? zc : n, false};
 }
 
 static dim3 correct_grid(int n, bool fp32) {
@@ -286,7 +288,7 @@ struct CorrArgs {
     int zc, xcd;
 };
 
-template <typename T, int MX, int MY, int U>
+template <typename T, int MX, int MY, int U, bool ROWS = false>
 __global__ __launch_bounds__(MX * MY)
 void k_correct(CorrArgs<T> one, const CorrArgs<T>* __restrict__ tab, int nbox) {
     const Blk blk = launch_blk(nbox);
@@ -346,107 +348,15 @@ void k_correct(CorrArgs<T> one, const CorrArgs<T>* __restrict__ tab, int nbox) {
     }
     su = wave_sum(su); sv = wave_sum(sv); sw = wave_sum(sw);
     mu_ = wave_max(mu_); mv_ = wave_max(mv_); mw_ = wave_max(mw_);
-    const int wv = tid >> 6;
-    if ((tid & 63) == 0) {
-        red[0][wv] = su; red[1][wv] = sv; red[2][wv] = sw;
-        red[3][wv] = mu_; red[4][wv] = mv_; red[5][wv] = mw_;
-    }
-    __syncthreads();
-    if (tid < 6) {
-        const int f = tid;
-        double r = red[f][0];
-        for (int t = 1; t < NT / 64; t++) r = (f < 3) ? r + red[f][t] : fmax(r, red[f][t]);
-        // partials in tile order, so the reduction order does not depend on
-        // the workgroup order (xcd_tile)
-        const size_t b = ((size_t)tbz * blk.ny + tby) * blk.nx + tbx;
-        partials[b * 6 + f] = r;
-    }
-}
-
-// The same with the column marched one plane at a time, p(z-1) of the column
-// in a register and the plane's p with a one-point halo at -x and -y in LDS.
-template <typename T, int CMX>
-__global__ __launch_bounds__(CO_NT)
-void k_correct_march(CorrArgs<T> one, const CorrArgs<T>* __restrict__ tab, int nbox) {
-    const Blk blk = launch_blk(nbox);
-    CorrArgs<T> A = one;
-    if (tab) A = tab[blk.box];
-    const MHIT_GLOBAL double* __restrict__ us = gmem(A.us);
-    const MHIT_GLOBAL double* __restrict__ vs = gmem(A.vs);
-    const MHIT_GLOBAL double* __restrict__ ws = gmem(A.ws);
-    const MHIT_GLOBAL T* __restrict__ p = gmem(A.p);
-    MHIT_GLOBAL double* __restrict__ u = gmem(A.u);
-    MHIT_GLOBAL double* __restrict__ v = gmem(A.v);
-    MHIT_GLOBAL double* __restrict__ w = gmem(A.w);
-    MHIT_GLOBAL double* __restrict__ partials = gmem(A.partials);
-    const Grid g = A.g;
-    const MHIT_GLOBAL DevScalars* __restrict__ S = gmem(A.S);
-    const int zc = A.zc, xcd = A.xcd;
-    constexpr int MX = CMX, MY = CO_NT / CMX, NT = MX * MY, W = MX + 1, H = MY + 1;
-    constexpr int NP = (W * H + NT - 1) / NT;
-    // p of the plane, x = -1..MX-1, y = -1..MY-1; two buffers, so that the
-    // next plane's commit needs no barrier after this plane's reads
-    __shared__ T sp2[2][W * H];
-    __shared__ double red[6][NT / 64];
-    const int n = g.n;
-    const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * MX + tx;
-    int tbx, tby, tbz;
-    xcd_tile(tbx, tby, tbz, blk, xcd);
-    const int i0 = tbx * MX, j0 = tby * MY, z0 = tbz * zc;
-    const int z1 = min(z0 + zc, n);
-    const int i = i0 + tx, j = j0 + ty;
-    const bool halted = S->halted != 0;
-    const bool live = !halted && i < n && j < n;
-    const double dtr = g.dt / g.rho;
-    double su = 0.0, sv = 0.0, sw = 0.0;
-    double mu_ = -INFINITY, mv_ = -INFINITY, mw_ = -INFINITY;
-    if (!halted) {
-        // in-plane offsets of the thread's halo points, fixed for the whole march
-        int off[NP];
-#pragma unroll
-        for (int t = 0; t < NP; t++) {
-            const int e = tid + t * NT;
-            const int lx = e % W, ly = e / W;
-            off[t] = (e < W * H) ? ((j0 + ly - 1 + n) % n) * n + (i0 + lx - 1 + n) % n : 0;
+    if constexpr (ROWS) {
+        // [chunk][row][64-cell segment]; the waves hold one segment each
+        if ((tid & 63) == 0) {
+            const double r[6] = {su, sv, sw, mu_, mv_, mw_};
+            const size_t b = ((size_t)tbz * n + j) * (n / 64) + i / 64;
+            for (int f = 0; f < 6; f++) partials[b * 6 + f] = r[f];
         }
-        T pf[NP];
-        auto fetch = [&](int k) {
-            const MHIT_GLOBAL T* __restrict__ pl = p + (size_t)k * n * n;
-#pragma unroll
-            for (int t = 0; t < NP; t++)
-                if ((W * H) % NT == 0 || tid + t * NT < W * H) pf[t] = pl[off[t]];
-        };
-        double pkm = live ? (double)p[idx3(i, j, wrap_m(z0, n), n)] : 0.0;
-        fetch(z0);
-        for (int k = z0; k < z1; k++) {
-            const size_t q = idx3(live ? i : 0, live ? j : 0, k, n);
-            double usq = 0.0, vsq = 0.0, wsq = 0.0;
-            if (live) { usq = ld_once(&us[q]); vsq = ld_once(&vs[q]); wsq = ld_once(&ws[q]); }   // in flight across the barrier
-            T* const sp = sp2[(k - z0) & 1];
-#pragma unroll
-            for (int t = 0; t < NP; t++) {
-                const int e = tid + t * NT;
-                if (e < W * H) sp[e] = pf[t];
-            }
-            lds_sync();
-            if (k + 1 < z1) fetch(k + 1);
-            if (live) {
-                const int c = (ty + 1) * W + tx + 1;
-                const double pc = (double)sp[c];
-                const double uu = usq - dtr * (pc - (double)sp[c - 1]) * g.dxi;
-                const double vv = vsq - dtr * (pc - (double)sp[c - W]) * g.dxi;
-                const double ww = wsq - dtr * (pc - pkm) * g.dxi;
-                st_once(&u[q], uu); st_once(&v[q], vv); st_once(&w[q], ww);
-                su += uu; sv += vv; sw += ww;
-                mu_ = fmax(mu_, uu); mv_ = fmax(mv_, vv); mw_ = fmax(mw_, ww);
-                pkm = pc;
-            }
-            // (the next commit goes to the other buffer; the one read here
-            // is written again only after the next plane's barrier)
-        }
+        return;
     }
-    su = wave_sum(su); sv = wave_sum(sv); sw = wave_sum(sw);
-    mu_ = wave_max(mu_); mv_ = wave_max(mv_); mw_ = wave_max(mw_);
     const int wv = tid >> 6;
     if ((tid & 63) == 0) {
         red[0][wv] = su; red[1][wv] = sv; red[2][wv] = sw;
@@ -475,10 +385,10 @@ static CorrArgs<T> corr_args(mhit_ctx* c) {
     a.S = c->S;
     const CorrShape sh = correct_shape(c->n, c->fp32);
     a.zc = sh.zc;
-    // XCD tile order where p's neighbours then hit in the same L2: the march
-    // (1.39 -> 1.36 ms at 512^3) and small boxes (96^3 10.9 against 11.3 us);
-    // the partials are indexed by tile, so the order changes no bit
-    a.xcd = sh.march || c->n < 192;
+    // XCD tile order for small boxes (96^3 10.9 against 11.3 us, 512^3 FP32
+    // 1.24 against 1.17 ms); the partials are indexed by tile, so the order
+    // changes no bit
+    a.xcd = c->n < 192;
     return a;
 }
 
@@ -490,8 +400,10 @@ static void go_correct(int n, const CorrArgs<T>& one, const CorrArgs<T>* tab, in
     grid.z *= nb;
     const dim3 block(sh.mx, sh.my, 1);
     if constexpr (F32) {
-        if (sh.march) {
-            k_correct_march<T, 64><<<grid, block, 0, st>>>(one, tab, nb);
+        if (sh.rows) {
+            if (sh.mx == 128) k_correct<T, 128, 2, 2, true><<<grid, block, 0, st>>>(one, tab, nb);
+            else if (n >= 512) k_correct<T, 256, 1, 2, true><<<grid, block, 0, st>>>(one, tab, nb);
+            else k_correct<T, 256, 1, 8, true><<<grid, block, 0, st>>>(one, tab, nb);
             return;
         }
     } else {
@@ -542,17 +454,24 @@ int launch_correct_batch(mhit_ctx* const* boxes, int nb, ArgArena& arena, hipStr
 // (998-1002, max(u - m) = max(u) - m as rounding is monotone), CFL
 // (1003-1006), AB2 switch (801-802).  One workgroup, fixed reduction order:
 // thread t adds up partials t, t + 1024, ..., then a tree over the threads.
-// Above kFinMost partials (the FP64 sweeps of large boxes) k_fin_parts first
-// adds up runs of kFinPart of them.
-constexpr int kFinMost = 4096, kFinPart = 64;
+// k_fin_rows first makes those 1024 sums from row sums (the FP32 sweeps of
+// large boxes), and above kFinMost partials (the FP64 ones) k_fin_parts
+// first adds up runs of kFinPart: one workgroup alone takes 16 us for the
+// 16,384 partials of 512^3.
+constexpr int kFinMost = 4096, kFinPart = 64, kFinRuns = 1024;
 
-static int fin_parts(int n, bool fp32) {
-    const int nb = correct_block_count(n, fp32);
-    return !fp32 && nb > kFinMost ? div_up(nb, kFinPart) : 0;
-}
+// partials of the correction's workgroups (waves, for row sums)
 int correct_block_count(int n, bool fp32) {
+    const CorrShape s = correct_shape(n, fp32);
+    if (s.rows) return (n / 64) * n * div_up(n, s.zc);
     const dim3 g = correct_grid(n, fp32);
     return (int)(g.x * g.y * g.z);
+}
+// sums that k_finalize starts from instead of the partials (0: none)
+static int fin_parts(int n, bool fp32) {
+    const int nb = correct_block_count(n, fp32);
+    if (correct_shape(n, fp32).rows) return std::min(kFinRuns, nb / 8);
+    return nb > kFinMost ? div_up(nb, kFinPart) : 0;
 }
 // space for the partials, in doubles: the correction's, then their sums
 size_t correct_partials(int n, bool fp32) {
@@ -582,6 +501,32 @@ void k_fin_parts(FinArgs one, const FinArgs* __restrict__ tab) {
         const double r = f < 3 ? wave_sum(x) : wave_max(x);
         if ((threadIdx.x & 63) == 0) partials[(size_t)(A.nblocks + run) * 6 + f] = r;
     }
+}
+
+// The row sums to the sums of the kFinRuns interleaved runs of 8-row tiles:
+// tile b is segment b % (n/64) of rows 8 b' ... 8 b' + 7, b' = b / (n/64)
+// (chunk by chunk), its rows are added up first to last, and run t holds
+// tiles t, t + kFinRuns, ...  A thread per run and component.
+__global__ __launch_bounds__(256)
+void k_fin_rows(FinArgs one, const FinArgs* __restrict__ tab) {
+    FinArgs A = one;
+    if (tab) A = tab[blockIdx.y];
+    const int q = blockIdx.x * 256 + threadIdx.x, t = q / 6, f = q - 6 * t;
+    if (t >= A.nparts) return;
+    MHIT_GLOBAL double* partials = gmem(A.partials);
+    const int nx = A.g.n / 64, tiles = A.nblocks / 8;
+    double r = f < 3 ? 0.0 : -INFINITY;
+#pragma unroll 2
+    for (int b = t; b < tiles; b += kFinRuns) {
+        const MHIT_GLOBAL double* row = partials + ((size_t)(b / nx) * 8 * nx + b % nx) * 6 + f;
+        double x[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) x[j] = row[(size_t)j * nx * 6];
+#pragma unroll
+        for (int j = 1; j < 8; j++) x[0] = f < 3 ? x[0] + x[j] : fmax(x[0], x[j]);
+        r = f < 3 ? r + x[0] : fmax(r, x[0]);
+    }
+    if (!gmem(A.S)->halted) partials[(size_t)(A.nblocks + t) * 6 + f] = r;
 }
 
 // One workgroup per box (blockIdx.x is the box of a batched launch).
@@ -647,14 +592,16 @@ static FinArgs fin_args(mhit_ctx* c) {
     return a;
 }
 
-static void go_finalize(const FinArgs& one, const FinArgs* tab, int nb, int nparts, hipStream_t st) {
-    if (nparts) k_fin_parts<<<dim3(div_up(nparts, 4), nb), 256, 0, st>>>(one, tab);
+static void go_finalize(mhit_ctx* c, const FinArgs& one, const FinArgs* tab, int nb, hipStream_t st) {
+    if (one.nparts && correct_shape(c->n, c->fp32).rows)
+        k_fin_rows<<<dim3(div_up(one.nparts * 6, 256), nb), 256, 0, st>>>(one, tab);
+    else if (one.nparts)
+        k_fin_parts<<<dim3(div_up(one.nparts, 4), nb), 256, 0, st>>>(one, tab);
     k_finalize<<<nb, 1024, 0, st>>>(one, tab);
 }
 
 int launch_finalize(mhit_ctx* c) {
-    const FinArgs a = fin_args(c);
-    go_finalize(a, nullptr, 1, a.nparts, c->stream);
+    go_finalize(c, fin_args(c), nullptr, 1, c->stream);
     prof_mark(c, ST_FINALIZE);
     MHIT_HIP_TRY(hipGetLastError());
     return MHIT_OK;
@@ -662,14 +609,16 @@ int launch_finalize(mhit_ctx* c) {
 
 int launch_finalize_batch(mhit_ctx* const* boxes, int nb, ArgArena& arena, hipStream_t st) {
     std::vector<FinArgs> t(nb);
-    int nparts = 0;
     for (int b = 0; b < nb; b++) {
         t[b] = fin_args(boxes[b]);
-        nparts = std::max(nparts, t[b].nparts);
+        if (boxes[b]->n != boxes[0]->n || boxes[b]->fp32 != boxes[0]->fp32) {
+            set_error("batched finalize: boxes differ in size or precision");
+            return MHIT_ERR_ARG;
+        }
     }
     const FinArgs* tab = arena.put(t.data(), nb);
     if (!tab) { set_error("batched launch: argument arena full"); return MHIT_ERR_STATE; }
-    go_finalize(t[0], tab, nb, nparts, st);
+    go_finalize(boxes[0], t[0], tab, nb, st);
     MHIT_HIP_TRY(hipGetLastError());
     return MHIT_OK;
 }
