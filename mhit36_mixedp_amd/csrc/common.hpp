@@ -142,6 +142,8 @@ __device__ __forceinline__ Blk launch_blk(int nbox) {
 // in memory) are generic to the compiler, which then emits flat memory
 // instructions; gmem() states that they point to global memory.
 #define MHIT_GLOBAL __attribute__((address_space(1)))
+// tables that no kernel writes: uniform reads go through the scalar cache
+#define MHIT_CONST __attribute__((address_space(4)))
 template <typename T>
 __device__ __forceinline__ MHIT_GLOBAL T* gmem(T* p) { return (MHIT_GLOBAL T*)p; }
 
