@@ -511,7 +511,7 @@ int mhit_create(const mhit_params* P, mhit_ctx** out) {
                                          &c->normz, &c->fxst, &c->fyst, &c->fzst});
     }
     for (double** f : fields)
-        if ((rc = dmalloc(f, N3))) return fail(rc);
+        if ((rc = dmalloc(f, N3 + kSink))) return fail(rc);
     const size_t H = n / 2;
     const size_t csz = c->fp32 ? sizeof(float2) : sizeof(double2);
     const size_t rsz = c->fp32 ? sizeof(float) : sizeof(double);

@@ -12,6 +12,12 @@
 
 struct mhit_dump_state;   // dump.hip
 
+namespace mhit {
+// Elements behind the n^3 of every field, where the ACDI pass puts what a
+// lane has computed for no cell of its own (march.hip); a workgroup's size
+constexpr size_t kSink = 1024;
+}
+
 struct mhit_ctx {
     mhit_params P;
     int n = 0;

@@ -35,6 +35,23 @@ __device__ __forceinline__ int wrapk(int k, int n) { return k < 0 ? k + n : (k >
 __device__ __forceinline__ int ring3(int k) { return ((k % 3) + 3) % 3; }
 __device__ __forceinline__ int ring4(int k) { return ((k % 4) + 4) % 4; }
 
+// Element of a field at a byte offset.  With a uniform base and an unsigned
+// 32-bit offset the address is a scalar pair and one register per lane
+// (a field of 512^3 doubles, the largest size, and its sink stay below 2^32
+// bytes).
+template <typename T>
+__device__ __forceinline__ MHIT_GLOBAL T* at_byte(MHIT_GLOBAL T* base, unsigned off) {
+    return (MHIT_GLOBAL T*)((MHIT_GLOBAL char*)base + off);
+}
+template <typename T>
+__device__ __forceinline__ const MHIT_GLOBAL T* at_byte(const MHIT_GLOBAL T* base, unsigned off) {
+    return (const MHIT_GLOBAL T*)((const MHIT_GLOBAL char*)base + off);
+}
+// Hides a value from the optimiser's view of the loop around it: without
+// this the compiler adds a loop-invariant offset to the field's base outside
+// the plane loop and keeps the 64-bit sum of every array in registers.
+__device__ __forceinline__ void opaque(unsigned& x) { asm("" : "+v"(x)); }
+
 // =====================================================================
 // NS + CSF + AB2 + divergence of u*
 // =====================================================================
@@ -372,6 +389,19 @@ void k_ns_march(NsArgs<TD> one, const NsArgs<TD>* __restrict__ tab, int nbox) {
 // Tile: TMX columns by TMY rows (Tuning::ac_my: 64 x 16, 64 x 8, 96 x 10 or
 // 32 x 32); z chunk: Tuning::ac_mz.  phi ring with a one-point halo, psi
 // ring with two.
+// Bound: memory.  The pass reads five fields and writes two, and what cost
+// it time was waiting.  Vector loads and stores complete in the order in
+// which they were issued, and a wave can wait for an older one with younger
+// ones in flight only where the compiler knows how many those are.  So every
+// plane issues the same loads and stores on every lane: the fetch of the
+// next plane, then the two stores, then the own column of the next plane.
+// Lanes without a cell of their own store to the kSink elements behind the
+// field, and a chunk fetches one plane that it does not use.  Before, with
+// stores and loads under conditions, each plane waited for all of them: ms
+// with / without conditions (FP32 Poisson, multiphase) 512^3 1.68 / 1.43
+// (5.3 TB/s of counted traffic), 256^3 0.220 / 0.198, 192^3 0.100 / 0.087, 128^3
+// 0.0370 / 0.0344, 96^3 0.0238 / 0.0235.  The 32-bit offsets took the kernel
+// from 124 to 96 registers.
 
 struct AcdiArgs {
     double* phi_out;
@@ -411,8 +441,10 @@ void k_acdi_march(AcdiArgs one, const AcdiArgs* __restrict__ tab, int nbox) {
     const int i0 = tbx * MX, j0 = tby * MY;
     const int z0 = tbz * zc;
     const int z1 = min(z0 + zc, n);
-    const int i = i0 + tx, j = j0 + ty;
-    const bool live = i < n && j < n;
+    // the cell, or its periodic image past the domain edge, whose results go
+    // to the sink behind the field
+    const int i = wrapn(i0 + tx, n), j = wrapn(j0 + ty, n);
+    const bool live = i0 + tx < n && j0 + ty < n;
     const double m0 = S->mean[0], m1 = S->mean[1], m2 = S->mean[2];
     const double alpha = S->alpha, beta = S->beta;
     const double gamma = 1.0 * S->gumax;               // main.f90:536
@@ -422,20 +454,22 @@ void k_acdi_march(AcdiArgs one, const AcdiArgs* __restrict__ tab, int nbox) {
     // phi of one plane in flight: global -> registers
     constexpr int NPL = (H2 * W2 + NT - 1) / NT;
     const size_t plane = (size_t)n * n;
-    // in-plane offsets of the thread's halo points, fixed for the whole march
-    int poff[NPL];
+    // in-plane byte offsets of the thread's halo points, fixed for the march
+    unsigned poff[NPL];
 #pragma unroll
     for (int t = 0; t < NPL; t++) {
         const int e = tid + t * NT;
         const int lx = e % W2, ly = e / W2;
-        poff[t] = (e < H2 * W2) ? wrapn(j0 - 2 + ly, n) * n + wrapn(i0 - 2 + lx, n) : 0;
+        poff[t] = (e < H2 * W2) ? 8u * (wrapn(j0 - 2 + ly, n) * n + wrapn(i0 - 2 + lx, n)) : poff[0];
     }
     struct Plane { double p[NPL]; };
     auto fetch = [&](int k, Plane& r) {
         const MHIT_GLOBAL double* __restrict__ pl = phi + (size_t)wrapk(k, n) * plane;
 #pragma unroll
-        for (int t = 0; t < NPL; t++)
-            if ((H2 * W2) % NT == 0 || tid + t * NT < H2 * W2) r.p[t] = pl[poff[t]];
+        for (int t = 0; t < NPL; t++) {
+            opaque(poff[t]);
+            r.p[t] = *at_byte(pl, poff[t]);
+        }
     };
     // registers -> psi ring (halo 2) and phi ring (halo 1), main.f90:522-534
     auto commit = [&](int k, const Plane& r) {
@@ -540,35 +574,33 @@ void k_acdi_march(AcdiArgs one, const AcdiArgs* __restrict__ tab, int nbox) {
     fz_0 = fluxes(z0, bf);
     lds_sync();
 
-    double wk = 0.0;
-    if (live) wk = w[idx3(i, j, z0, n)] - m2;
-    // velocity faces and AB2 history of the own column, a plane ahead (loaded
-    // in the plane that uses them, every plane waited for them: 1.70 -> 1.63
-    // ms at 512^3, 5.1 TB/s of counted traffic, what a march with this many
-    // streams reaches without any stencil)
-    struct Own { double u, up, v, vp, wp, ro; };
-    auto own = [&](int k, Own& r) {
-        if (!live) return;
-        const size_t q = idx3(i, j, k, n);
-        r.u = u[q];
-        r.up = u[idx3(wrap_p(i, n), j, k, n)];
-        r.v = v[q];
-        r.vp = v[idx3(i, wrap_p(j, n), k, n)];
-        r.wp = w[idx3(i, j, wrap_p(k, n), n)];
-        r.ro = rphi_o[q];
+    // velocity faces and AB2 history of the own column, reloaded as soon as
+    // the plane has used them
+    unsigned o = 8u * (j * n + i), ox = 8u * (j * n + wrap_p(i, n)), oy = 8u * (wrap_p(j, n) * n + i);
+    const unsigned sink = 8u * ((unsigned)n * (unsigned)plane + tid);
+    double wk = *at_byte(w + z0 * plane, o) - m2;
+    struct Own { double u, up, v, vp, wp, ro; } own;
+    auto fetch_own = [&](int k) {
+        const size_t b = (size_t)wrapk(k, n) * plane;
+        opaque(o);
+        opaque(ox);
+        opaque(oy);
+        own.u = *at_byte(u + b, o);
+        own.up = *at_byte(u + b, ox);
+        own.v = *at_byte(v + b, o);
+        own.vp = *at_byte(v + b, oy);
+        own.wp = *at_byte(w + wrapk(k + 1, n) * plane, o);
+        own.ro = *at_byte((const MHIT_GLOBAL double*)rphi_o + b, o);
     };
-    Own on;
-    own(z0, on);
+    fetch_own(z0);
     for (int k = z0; k < z1; k++) {
-        const size_t q = idx3(live ? i : 0, live ? j : 0, k, n);
-        const Own o = on;
+        const unsigned q = live ? k * (8u * (unsigned)plane) + o : sink;
         commit(k + 2, nx);
         lds_sync();
-        if (k + 3 <= z1 + 1) fetch(k + 3, nx);   // next plane in flight during the compute
-        if (k + 1 < z1) own(k + 1, on);
+        fetch(k + 3, nx);   // next plane in flight during the compute
         fz_p1 = fluxes(k + 1, bf ^ 1);
-        if (live) {
-            const double uc = o.u - m0, up = o.up - m0, vc = o.v - m1, vp = o.vp - m1, wp = o.wp - m2;
+        {
+            const double uc = own.u - m0, up = own.up - m0, vc = own.v - m1, vp = own.vp - m1, wp = own.wp - m2;
             const double pc = PH(k, tx, ty);
             const double pxp = PH(k, tx + 1, ty), pxm = PH(k, tx - 1, ty);
             const double pyp = PH(k, tx, ty + 1), pym = PH(k, tx, ty - 1);
@@ -588,9 +620,10 @@ void k_acdi_march(AcdiArgs one, const AcdiArgs* __restrict__ tab, int nbox) {
                                 (Fy[(ty + 2) * MX + tx] - Fy[ty * MX + tx])) + (fz_p1 - fz_m1);
             const double r = gamma * (ced * lap - hdx * shp) - hdx * conv;
             // P5 AB2, main.f90:625-626
-            st_once(&phi_out[q], pc + dt * (alpha * r - beta * o.ro));
-            st_once(&rphi_o[q], r);
+            st_once(at_byte(phi_out, q), pc + dt * (alpha * r - beta * own.ro));
+            st_once(at_byte(rphi_o, q), r);
             wk = wp;
+            fetch_own(k + 1);
         }
         fz_m1 = fz_0;
         fz_0 = fz_p1;
