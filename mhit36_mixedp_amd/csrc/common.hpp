@@ -146,6 +146,22 @@ __device__ __forceinline__ Blk launch_blk(int nbox) {
 #define MHIT_CONST __attribute__((address_space(4)))
 template <typename T>
 __device__ __forceinline__ MHIT_GLOBAL T* gmem(T* p) { return (MHIT_GLOBAL T*)p; }
+// Element of a field at a byte offset.  With a uniform base and an unsigned
+// 32-bit offset the address is a scalar pair and one register per lane
+// (a field of 512^3 doubles, the largest size, and its sink stay below 2^32
+// bytes).
+template <typename T>
+__device__ __forceinline__ MHIT_GLOBAL T* at_byte(MHIT_GLOBAL T* base, unsigned off) {
+    return (MHIT_GLOBAL T*)((MHIT_GLOBAL char*)base + off);
+}
+template <typename T>
+__device__ __forceinline__ const MHIT_GLOBAL T* at_byte(const MHIT_GLOBAL T* base, unsigned off) {
+    return (const MHIT_GLOBAL T*)((const MHIT_GLOBAL char*)base + off);
+}
+// Hides a value from the optimiser: without this the compiler adds a
+// loop-invariant offset to a field's base outside the loop, or once for the
+// load and the store of an element, and keeps the 64-bit sums in registers.
+__device__ __forceinline__ void opaque(unsigned& x) { asm("" : "+v"(x)); }
 
 // Load / store of a two-component HIP vector (float2, double2) through a
 // global pointer: the vector type's operators take generic references, so

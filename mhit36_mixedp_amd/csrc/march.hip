@@ -35,23 +35,6 @@ __device__ __forceinline__ int wrapk(int k, int n) { return k < 0 ? k + n : (k >
 __device__ __forceinline__ int ring3(int k) { return ((k % 3) + 3) % 3; }
 __device__ __forceinline__ int ring4(int k) { return ((k % 4) + 4) % 4; }
 
-// Element of a field at a byte offset.  With a uniform base and an unsigned
-// 32-bit offset the address is a scalar pair and one register per lane
-// (a field of 512^3 doubles, the largest size, and its sink stay below 2^32
-// bytes).
-template <typename T>
-__device__ __forceinline__ MHIT_GLOBAL T* at_byte(MHIT_GLOBAL T* base, unsigned off) {
-    return (MHIT_GLOBAL T*)((MHIT_GLOBAL char*)base + off);
-}
-template <typename T>
-__device__ __forceinline__ const MHIT_GLOBAL T* at_byte(const MHIT_GLOBAL T* base, unsigned off) {
-    return (const MHIT_GLOBAL T*)((const MHIT_GLOBAL char*)base + off);
-}
-// Hides a value from the optimiser's view of the loop around it: without
-// this the compiler adds a loop-invariant offset to the field's base outside
-// the plane loop and keeps the 64-bit sum of every array in registers.
-__device__ __forceinline__ void opaque(unsigned& x) { asm("" : "+v"(x)); }
-
 // =====================================================================
 // NS + CSF + AB2 + divergence of u*
 // =====================================================================

@@ -467,6 +467,23 @@ __device__ __forceinline__ void cols_body(const ColArgs<T>& A, const int bxi, co
     };
 
     static_assert((N * C) % NT == 0, "column tile must be a multiple of the workgroup");
+    // Element a0 + a of the thread's column, o0 = a0 sa + c sc.  The z pass
+    // addresses it as a uniform base and a 32-bit byte offset: eight 64-bit
+    // addresses kept from the loads to the stores took it to 78 registers
+    // (FP32, 512^3) and three workgroups to a CU, without them it has 62 and
+    // four (512^3 297 -> 277 us, 384^3 145 -> 130, 192^3 22.9 -> 21.5; the
+    // arithmetic of two transforms is as long as the traffic, so what is in
+    // flight decides).  The y passes have registers to spare and measured
+    // 185 -> 189 us, so they keep pointers.
+    auto elem = [&](size_t o0, int a) -> MHIT_GLOBAL V* {
+        if constexpr (MODE == 2) {
+            unsigned off = (unsigned)sizeof(V) * (unsigned)o0;
+            opaque(off);
+            return at_byte(g + (size_t)a * sa, off);
+        } else {
+            return g + (o0 + (size_t)a * sa);
+        }
+    };
     // Wavefront form: N = 8 M 8 (M = 1, 2, 4, 8), eight columns, N/8
     // threads per column, thread t = b + 8 w of column c in lane 8 b + c of
     // wave w.  With n = n0 + 8 n1 + 8M n2 the thread holds x[t + 8M r], so
@@ -496,7 +513,7 @@ __device__ __forceinline__ void cols_body(const ColArgs<T>& A, const int bxi, co
             for (int r = 0; r < 8; r++) v[r] = ld(g + (size_t)spec_k(r) * sa + c * sc);
         } else {
 #pragma unroll
-            for (int r = 0; r < 8; r++) v[r] = ld(g + (size_t)(t + r * TPC) * sa + c * sc);
+            for (int r = 0; r < 8; r++) v[r] = ld(elem(t * sa + c * sc, r * TPC));
         }
         stage_twiddles<V, N, NT>(stw, tw, tid);
         if constexpr (MODE == 2) {
@@ -594,7 +611,7 @@ __device__ __forceinline__ void cols_body(const ColArgs<T>& A, const int bxi, co
             for (int r = 0; r < 8; r++) st(g + (size_t)spec_k(r) * sa + c * sc, v[r]);
         } else {
 #pragma unroll
-            for (int r = 0; r < 8; r++) st(g + (size_t)(t + r * TPC) * sa + c * sc, v[r]);
+            for (int r = 0; r < 8; r++) st(elem(t * sa + c * sc, r * TPC), v[r]);
         }
         return;
     }
@@ -612,7 +629,7 @@ __device__ __forceinline__ void cols_body(const ColArgs<T>& A, const int bxi, co
         const int c = tid % C, t = tid / C;
         V v[8];
 #pragma unroll
-        for (int r = 0; r < 8; r++) v[r] = ld(g + (size_t)(t + r * TPC) * sa + c * sc);
+        for (int r = 0; r < 8; r++) v[r] = ld(elem(t * sa + c * sc, r * TPC));
         stage_twiddles<V, N, NT>(stw, tw, tid);
         // per-axis k^2, staged with the data
         if constexpr (MODE == 2) {
@@ -657,7 +674,7 @@ __device__ __forceinline__ void cols_body(const ColArgs<T>& A, const int bxi, co
         }
         if (halted) return;
 #pragma unroll
-        for (int r = 0; r < 8; r++) st(g + (size_t)(t + r * TPC) * sa + c * sc, v[r]);
+        for (int r = 0; r < 8; r++) st(elem(t * sa + c * sc, r * TPC), v[r]);
         return;
     }
     {
@@ -894,9 +911,9 @@ struct PoissonPasses {
     }
     // Default z width, FP32: half the y pass's columns per workgroup
     // (64-byte row segments): the two FFTs of the z pass make it the
-    // longest-running column kernel, and smaller workgroups (two per CU at
-    // its register count) hide its barriers better (0.38 -> 0.33 ms at
-    // 512^3).  FP64 keeps 8 columns (128-byte segments; 4 columns measured
+    // longest-running column kernel, and smaller workgroups (four per CU at
+    // 512^3, against two of twice the size) hide its barriers better (0.38 ->
+    // 0.33 ms at 512^3 when both sizes had half as many resident).  FP64 keeps 8 columns (128-byte segments; 4 columns measured
     // 0.84 vs 0.55 ms).
     template <int MODE>
     static int z_pass(Boxes bx, int nb, ArgArena* ar, hipStream_t st) {
