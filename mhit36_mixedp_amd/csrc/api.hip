@@ -523,7 +523,7 @@ int mhit_create(const mhit_params* P, mhit_ctx** out) {
     if ((rc = dmalloc(&c->mysin, 3 * (size_t)(n + 1)))) return fail(rc);
     c->mycos = c->mysin + (n + 1);
     c->xext = c->mysin + 2 * (n + 1);
-    c->npart_blocks = correct_block_count(n, c->fp32);
+    c->npart_blocks = correct_block_count(n, c->fp32, 1);
     if ((rc = dmalloc(&c->partials, correct_partials(n, c->fp32)))) return fail(rc);
     c->ndiag_blocks = diag_block_count(n);
     const size_t ndp = std::max((size_t)c->ndiag_blocks * 8, (size_t)spectrum_blocks(n) * shells_used(n));

@@ -262,7 +262,7 @@ int launch_finalize(mhit_ctx* c);
 int launch_correct_batch(mhit_ctx* const* boxes, int nb, ArgArena& arena, hipStream_t st);
 int launch_finalize_batch(mhit_ctx* const* boxes, int nb, ArgArena& arena, hipStream_t st);
 int launch_diag(mhit_ctx* c, double* host_out /* 8 values */);
-int correct_block_count(int n, bool fp32);
+int correct_block_count(int n, bool fp32, int nb);
 size_t correct_partials(int n, bool fp32);   // doubles in mhit_ctx::partials
 int diag_block_count(int n);
 int launch_copy_probe(mhit_ctx* c, const void* src, void* dst, size_t bytes);

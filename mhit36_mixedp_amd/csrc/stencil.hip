@@ -258,9 +258,13 @@ int launch_ns(mhit_ctx* c) {
 // multiple of 256) over the order's chunk, 512^3 1.27 -> 1.22 ms, 384^3 0.59
 // -> 0.54, 256^3 0.172 -> 0.158 (5.5 TB/s) against the march; a wave writes
 // its row's sums and k_fin_rows (4 us) adds them up as an 8-row tile would.
+// The rows start where a launch covers as many cells as 256^3, so that an
+// ensemble's batches of 128^3 take them too (eight planes in flight: 16 x
+// 64^3 + 16 x 96^3 + 16 x 128^3 2.44 -> 2.36 ms per step, 16 x 128^3 1.51 ->
+// 1.48; 128^3 alone 0.109 -> 0.113, so not there).
 constexpr int CO_NT = 512;                    // threads per workgroup of the 8-row tile
 struct CorrShape { int mx, my, zc; bool rows; };
-static CorrShape correct_shape(int n, bool fp32) {
+static CorrShape correct_shape(int n, bool fp32, int nb) {
     if (!fp32 && n >= 64) return {n >= 256 ? 128 : (n % 64 == 0 ? 64 : 32), n % 64 == 0 ? 4 : 16,
                                   n >= 256 ? 2 : 4, false};
     const int mx = (n > 64 && n % 64 != 0 && n % 32 == 0) ? 32 : 64, my = CO_NT / mx;
@@ -268,12 +272,13 @@ static CorrShape correct_shape(int n, bool fp32) {
     const long long tiles = (long long)div_up(n, mx) * div_up(n, my);
     int zc = n >= 512 ? 16 : 32;
     while (n < 512 && zc > 2 && tiles * div_up(n, zc) < 256) zc /= 2;
-    if (n >= 256 && n % 128 == 0) return {n % 256 == 0 ? 256 : 128, n % 256 == 0 ? 1 : 2, zc, true};
+    if (n % 128 == 0 && (long long)n * n * n * nb >= 256LL * 256 * 256)
+        return {n % 256 == 0 ? 256 : 128, n % 256 == 0 ? 1 : 2, zc, true};
     return {mx, my, zc < n ? zc : n, false};
 }
 
-static dim3 correct_grid(int n, bool fp32) {
-    const CorrShape s = correct_shape(n, fp32);
+static dim3 correct_grid(int n, bool fp32, int nb) {
+    const CorrShape s = correct_shape(n, fp32, nb);
     return dim3(div_up(n, s.mx), div_up(n, s.my), div_up(n, s.zc));
 }
 
@@ -383,8 +388,7 @@ static CorrArgs<T> corr_args(mhit_ctx* c) {
     a.partials = c->partials;
     a.g = c->g;
     a.S = c->S;
-    const CorrShape sh = correct_shape(c->n, c->fp32);
-    a.zc = sh.zc;
+    a.zc = correct_shape(c->n, c->fp32, 1).zc;   // the same for any nb
     // XCD tile order for small boxes (96^3 10.9 against 11.3 us, 512^3 FP32
     // 1.24 against 1.17 ms); the partials are indexed by tile, so the order
     // changes no bit
@@ -395,13 +399,14 @@ static CorrArgs<T> corr_args(mhit_ctx* c) {
 template <typename T>
 static void go_correct(int n, const CorrArgs<T>& one, const CorrArgs<T>* tab, int nb, hipStream_t st) {
     constexpr bool F32 = sizeof(T) == 4;
-    const CorrShape sh = correct_shape(n, F32);
-    dim3 grid = correct_grid(n, F32);
+    const CorrShape sh = correct_shape(n, F32, nb);
+    dim3 grid = correct_grid(n, F32, nb);
     grid.z *= nb;
     const dim3 block(sh.mx, sh.my, 1);
     if constexpr (F32) {
         if (sh.rows) {
-            if (sh.mx == 128) k_correct<T, 128, 2, 2, true><<<grid, block, 0, st>>>(one, tab, nb);
+            if (n == 128) k_correct<T, 128, 2, 8, true><<<grid, block, 0, st>>>(one, tab, nb);
+            else if (sh.mx == 128) k_correct<T, 128, 2, 2, true><<<grid, block, 0, st>>>(one, tab, nb);
             else if (n >= 512) k_correct<T, 256, 1, 2, true><<<grid, block, 0, st>>>(one, tab, nb);
             else k_correct<T, 256, 1, 8, true><<<grid, block, 0, st>>>(one, tab, nb);
             return;
@@ -461,21 +466,23 @@ int launch_correct_batch(mhit_ctx* const* boxes, int nb, ArgArena& arena, hipStr
 constexpr int kFinMost = 4096, kFinPart = 64, kFinRuns = 1024;
 
 // partials of the correction's workgroups (waves, for row sums)
-int correct_block_count(int n, bool fp32) {
-    const CorrShape s = correct_shape(n, fp32);
+int correct_block_count(int n, bool fp32, int nb) {
+    const CorrShape s = correct_shape(n, fp32, nb);
     if (s.rows) return (n / 64) * n * div_up(n, s.zc);
-    const dim3 g = correct_grid(n, fp32);
+    const dim3 g = correct_grid(n, fp32, nb);
     return (int)(g.x * g.y * g.z);
 }
 // sums that k_finalize starts from instead of the partials (0: none)
-static int fin_parts(int n, bool fp32) {
-    const int nb = correct_block_count(n, fp32);
-    if (correct_shape(n, fp32).rows) return std::min(kFinRuns, nb / 8);
-    return nb > kFinMost ? div_up(nb, kFinPart) : 0;
+static int fin_parts(int n, bool fp32, int nb) {
+    const int parts = correct_block_count(n, fp32, nb);
+    if (correct_shape(n, fp32, nb).rows) return std::min(kFinRuns, parts / 8);
+    return parts > kFinMost ? div_up(parts, kFinPart) : 0;
 }
-// space for the partials, in doubles: the correction's, then their sums
+// space for the partials, in doubles: the correction's, then their sums, of
+// a box alone or in a launch of any number of boxes
 size_t correct_partials(int n, bool fp32) {
-    return (size_t)(correct_block_count(n, fp32) + fin_parts(n, fp32)) * 6;
+    auto need = [&](int nb) { return (size_t)(correct_block_count(n, fp32, nb) + fin_parts(n, fp32, nb)) * 6; };
+    return std::max(need(1), need(1 << 20));
 }
 
 struct FinArgs {
@@ -581,11 +588,11 @@ void k_finalize(FinArgs one, const FinArgs* __restrict__ tab) {
     }
 }
 
-static FinArgs fin_args(mhit_ctx* c) {
+static FinArgs fin_args(mhit_ctx* c, int nb) {
     FinArgs a;
     a.partials = c->partials;
-    a.nblocks = c->npart_blocks;
-    a.nparts = fin_parts(c->n, c->fp32);
+    a.nblocks = correct_block_count(c->n, c->fp32, nb);
+    a.nparts = fin_parts(c->n, c->fp32, nb);
     a.cfl_abort = c->P.cfl_abort;
     a.g = c->g;
     a.S = c->S;
@@ -593,7 +600,7 @@ static FinArgs fin_args(mhit_ctx* c) {
 }
 
 static void go_finalize(mhit_ctx* c, const FinArgs& one, const FinArgs* tab, int nb, hipStream_t st) {
-    if (one.nparts && correct_shape(c->n, c->fp32).rows)
+    if (one.nparts && correct_shape(c->n, c->fp32, nb).rows)
         k_fin_rows<<<dim3(div_up(one.nparts * 6, 256), nb), 256, 0, st>>>(one, tab);
     else if (one.nparts)
         k_fin_parts<<<dim3(div_up(one.nparts, 4), nb), 256, 0, st>>>(one, tab);
@@ -601,7 +608,7 @@ static void go_finalize(mhit_ctx* c, const FinArgs& one, const FinArgs* tab, int
 }
 
 int launch_finalize(mhit_ctx* c) {
-    go_finalize(c, fin_args(c), nullptr, 1, c->stream);
+    go_finalize(c, fin_args(c, 1), nullptr, 1, c->stream);
     prof_mark(c, ST_FINALIZE);
     MHIT_HIP_TRY(hipGetLastError());
     return MHIT_OK;
@@ -610,7 +617,7 @@ int launch_finalize(mhit_ctx* c) {
 int launch_finalize_batch(mhit_ctx* const* boxes, int nb, ArgArena& arena, hipStream_t st) {
     std::vector<FinArgs> t(nb);
     for (int b = 0; b < nb; b++) {
-        t[b] = fin_args(boxes[b]);
+        t[b] = fin_args(boxes[b], nb);
         if (boxes[b]->n != boxes[0]->n || boxes[b]->fp32 != boxes[0]->fp32) {
             set_error("batched finalize: boxes differ in size or precision");
             return MHIT_ERR_ARG;

@@ -54,3 +54,23 @@ def test_correction_mean_and_max(n, prec):
             assert abs(v.mean()) < 1e-13
             assert abs(d[m] - v0.mean()) < 1e-12
         assert d["gumax"] == max(v.max() for v in vel)
+
+
+@pytest.mark.parametrize("boxes", [7, 8, 9])
+def test_batched_correction_of_128(boxes):
+    """Batches of 128^3 below, at and above the size from which the
+    correction sweeps flat rows: the bits of each box stepped alone."""
+    from mhit36_mixedp_amd import Ensemble, Solver, default_params
+    print(f"[shapes] {boxes} x 128^3", flush=True)
+    p = [default_params(nx=128, phiflag=0, poisson_precision=1, dt=2e-4, mu=0.006) for _ in range(boxes)]
+    with Ensemble(p) as ens:
+        for b, box in enumerate(ens.boxes):
+            box.init_random_velocity(3 + b, kmax=4.0, urms=1.0)
+        ens.step(3)
+        for b in (0, boxes // 2, boxes - 1):
+            with Solver(p[b]) as s:
+                s.init_random_velocity(3 + b, kmax=4.0, urms=1.0)
+                s.step(3)
+                assert s.scalars() == ens.boxes[b].scalars(), b
+                for f in range(1, 4):
+                    assert np.array_equal(s.download_field(f), ens.boxes[b].download_field(f)), (b, f)
