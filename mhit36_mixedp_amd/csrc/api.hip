@@ -141,9 +141,10 @@ int chunk_planes(int n, long long tiles, int slots, int cap) {
 
 // Launch shapes by grid size, then MHIT_TUNE; mhit_autotune refines.
 // A box alone: 64 x 8 tiles up to 64^3, 64 x 16 above (less halo), and
-// 64 x 8 in the ACDI pass of 128^3 to 384^3, two workgroups to a CU (192^3
-// 0.468 -> 0.460 ms per step, 384^3 3.14 -> 3.11; 512^3 6.95 -> 6.98, so
-// not there); z chunks by chunk_planes.  Measured, ms per step, FP32
+// 64 x 8 in the ACDI pass below 256^3, two workgroups to a CU (against
+// 64 x 16, ms per step: 128^3 0.147 and 0.147, 192^3 0.450 and 0.452; from
+// 256^3 the halo costs more: 0.823 and 0.802, 384^3 2.82 and 2.82); z chunks
+// by chunk_planes.  Measured, ms per step, FP32
 // Poisson, single phase / multiphase, against chunks halved from
 // min(128, n/4) until there is a workgroup per CU: 96^3 0.081 / 0.114 at 6
 // planes -> 0.075 / 0.099 at 4 (240 instead of 160 workgroups); 192^3
@@ -167,7 +168,7 @@ void default_tuning(mhit_ctx* c, bool batched, bool env) {
     c->tune.ac_my = rows;
     c->tune.ns_mz = c->tune.ac_mz = std::min(128, n);
     if (!batched) {
-        if (rows == 16 && n >= 128 && n < 512) c->tune.ac_my = 8;
+        if (rows == 16 && n < 256) c->tune.ac_my = 8;
         auto tiles = [&](int my) { return (long long)div_up(n, tile_cols(my)) * div_up(n, my); };
         const int ac_slots = (c->tune.ac_my == 8 && n > 64) ? 2 * c->cus : c->cus;
         const int least = std::min(4, n);
