@@ -192,9 +192,13 @@ int mhit_set_ab2_state(mhit_ctx* ctx, double alpha, double beta, double gumax);
  * (fft_wave, and widths that move a pass to or from eight columns), which
  * changes rounding.                                                       */
 typedef struct mhit_tuning {
-    int32_t ns_mz;        /* z planes per workgroup, fused NS pass (fewer in
-                             a launch that would leave CUs without one)     */
-    int32_t ac_mz;        /* z planes per workgroup, fused ACDI pass        */
+    int32_t ns_mz;        /* z planes per workgroup, fused NS pass (n where
+                             that is less).  4, the default up to 96^3,
+                             stands for at most 4: a launch that would leave
+                             CUs without a workgroup takes fewer (1 up to
+                             32^3, 2 at 48^3 and 64^3).  Every other value is
+                             launched as it is                              */
+    int32_t ac_mz;        /* z planes per workgroup, fused ACDI pass: the same */
     int32_t xcd;          /* 1: XCD-aware workgroup order, fused passes (the
                              default up to 256^3 and in ensembles)          */
     int32_t sort_every;   /* tracer re-ordering period in steps (0: never)  */

@@ -139,6 +139,13 @@ int chunk_planes(int n, long long tiles, int slots, int cap) {
     return best;
 }
 
+// Planes per workgroup of a pass over nb boxes of n^3 in tiles of `my` rows:
+// zc, or fewer where that would leave CUs without a workgroup.
+int busy_chunk(int n, int my, int nb, int zc, int cus) {
+    const long long tiles = (long long)div_up(n, tile_cols(my)) * div_up(n, my) * nb;
+    return tiles * div_up(n, zc) < cus ? chunk_planes(n, tiles, cus, zc) : zc;
+}
+
 // Launch shapes by grid size, then MHIT_TUNE; mhit_autotune refines.
 // A box alone: 64 x 8 tiles up to 64^3, 64 x 16 above (less halo), and
 // 64 x 8 in the ACDI pass below 256^3, two workgroups to a CU (against
@@ -151,10 +158,10 @@ int chunk_planes(int n, long long tiles, int slots, int cap) {
 // 0.384 / 0.609 at 24 -> 0.325 / 0.460 at 28 (252 workgroups in one round
 // instead of 288 in two); 384^3 2.38 / 3.60 at 96 -> 2.16 / 3.11 at 55 (3.9
 // rounds instead of 2.25); 128^3 (8) and 256^3 (64) unchanged; 512^3 6.99
-// -> 6.97 at 256.  Launches that still leave CUs idle at 4 planes are
-// shortened further (pass_chunk in march.hip).  Boxes batched in an
-// ensemble: 64x16 tiles and min(n, 128) planes, which the ensemble then
-// shortens until its launches fill the GPU.
+// -> 6.97 at 256.  Boxes that would get fewer than kShortChunk planes (up to
+// 64^3) take that value, which the launch shortens (pass_chunk in march.hip).
+// Boxes batched in an ensemble: 64x16 tiles and min(n, 128) planes, which the
+// ensemble then shortens until its launches fill the GPU.
 void default_tuning(mhit_ctx* c, bool batched, bool env) {
     const int n = c->n;
     // 96 x 10 tiles where 64-column tiles would leave part of each row of
@@ -171,9 +178,8 @@ void default_tuning(mhit_ctx* c, bool batched, bool env) {
         if (rows == 16 && n < 256) c->tune.ac_my = 8;
         auto tiles = [&](int my) { return (long long)div_up(n, tile_cols(my)) * div_up(n, my); };
         const int ac_slots = (c->tune.ac_my == 8 && n > 64) ? 2 * c->cus : c->cus;
-        const int least = std::min(4, n);
-        c->tune.ns_mz = std::max(least, chunk_planes(n, tiles(rows), c->cus, 256));
-        c->tune.ac_mz = std::max(least, chunk_planes(n, tiles(c->tune.ac_my), ac_slots, 256));
+        c->tune.ns_mz = std::max(kShortChunk, chunk_planes(n, tiles(rows), c->cus, 256));
+        c->tune.ac_mz = std::max(kShortChunk, chunk_planes(n, tiles(c->tune.ac_my), ac_slots, 256));
     }
     // XCD tile order: neighbouring tiles of a box then share an XCD's L2.
     // Batched (the 64^3 / 96^3 / 128^3 ensemble 18.78-18.84k -> 18.87-

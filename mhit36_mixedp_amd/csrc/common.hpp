@@ -45,6 +45,10 @@ struct DevScalars {
 // DFT with a different operation order).  Defaults are set by grid size at
 // create; MHIT_TUNE="ns_mz=64,ac_mz=64,ns_my=16,ac_my=8,xcd=1,sort=10,fft=1,
 // ycols=16,zcols=8,xrows=8" overrides them.
+// A z chunk of kShortChunk planes is the one value a launch does not take as
+// it is: it takes fewer planes while CUs would have no workgroup (pass_chunk
+// in march.hip).  It is the default where less than that is best, up to 64^3.
+constexpr int kShortChunk = 4;
 struct Tuning {
     int ns_mz = 64;       // planes per workgroup, NS pass (set by grid size at create)
     int ac_mz = 64;       // planes per workgroup, ACDI pass (likewise)

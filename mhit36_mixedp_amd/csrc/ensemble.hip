@@ -194,12 +194,18 @@ static int enqueue_size_class(const std::vector<mhit_ctx*>& boxes, ArgArena& ar,
 // where n is not a multiple of 64) in XCD order and z
 // chunks of min(n, 128) planes, then chunks halved size class by size
 // class (the class with the longest chunks first, ties to the larger grid;
-// never below 8 planes) until the NS launches of one step hold at least
+// not below 8 planes) until the NS launches of one step hold at least
 // four workgroups per CU in total.  Measured on 16 boxes of one size: 64^3
 // 0.88 -> 0.30 ms per ensemble step (8-plane chunks), 96^3 1.57 -> 0.96 ms
-// (12), 128^3 2.52 -> 1.76 ms (32); the 16 x 64^3 + 16 x 96^3 + 16 x 128^3
-// mix, which fills the GPU already at full chunks through its concurrent
-// size classes, keeps 2.9 ms within 2%.  MHIT_TUNE overrides apply last.
+// (12), 128^3 2.52 -> 1.76 ms (32).  Last, a launch (the boxes of one size,
+// phase flag and precision) that would still leave CUs without a workgroup
+// by itself gets shorter chunks, down to one plane, also beside size classes
+// that would fill the GPU without it.  In the 16 x 64^3 + 16 x 96^3 + 16 x
+// 128^3 mix that takes 64^3 to 8 planes (2.34 ms at 64, 2.31 at 16, 2.28 at
+// 8, 2.39 at 1) and 96^3 to 32 (2.29 at 48, 2.28 at 32, 2.26 at 24).  A single
+// 64^3 box with drops goes to one plane: 1.51 ms beside 16 x 128^3 (1.50 at 8
+// planes, 1.63 at 64), 0.326 beside 6 x 96^3 (0.331 and 0.474).  MHIT_TUNE
+// overrides apply last.
 static void batched_shapes(const std::vector<mhit_ctx*>& boxes) {
     for (mhit_ctx* c : boxes) default_tuning(c, true, false);
     int cus = 0;
@@ -235,7 +241,14 @@ static void batched_shapes(const std::vector<mhit_ctx*>& boxes) {
         pick->second /= 2;
     }
     for (mhit_ctx* c : boxes) {
-        c->tune.ns_mz = c->tune.ac_mz = zc_of(c->n);
+        int ns = 0, ac = 0;   // boxes that share c's NS and ACDI launches
+        for (mhit_ctx* o : boxes) {
+            if (o->n != c->n) continue;
+            ac += o->P.phiflag != 0;
+            ns += (o->P.phiflag != 0) == (c->P.phiflag != 0) && o->fp32 == c->fp32;
+        }
+        c->tune.ns_mz = busy_chunk(c->n, c->tune.ns_my, ns, zc_of(c->n), cus);
+        c->tune.ac_mz = c->P.phiflag ? busy_chunk(c->n, c->tune.ac_my, ac, zc_of(c->n), cus) : c->tune.ns_mz;
         tuning_env(c);
     }
 }
@@ -510,9 +523,8 @@ int mhit_ensemble_autotune(mhit_ensemble* e, int steps, double* ms_per_step) {
         if (rc != MHIT_OK) break;
         mhit_ctx* c0 = cls[0];
         const int n = c0->n;
-        std::vector<int> zc = {c0->tune.ns_mz};
-        for (int z = n; z >= 8; z /= 2)
-            if (z != c0->tune.ns_mz) zc.push_back(z);
+        std::vector<int> zc;
+        for (int z = n; z >= 8; z /= 2) zc.push_back(z);
         auto widths = [&](int pass) {
             int w[3];
             const int k = fft_widths(n, c0->fp32, pass, w);
@@ -537,24 +549,32 @@ int mhit_ensemble_autotune(mhit_ensemble* e, int steps, double* ms_per_step) {
         };
         for (const Param& p : params) {
             if (rc != MHIT_OK) break;
-            if (p.cand.size() < 2) continue;
-            const int keep = c0->tune.*(p.field);
-            int best = keep;
-            double bms = best_ms;   // the current setting's time
-            for (int v : p.cand) {
-                if (v == keep) continue;
-                for (mhit_ctx* c : cls) {
-                    c->tune.*(p.field) = v;
-                    if (p.also) c->tune.*(p.also) = v;
+            if (p.cand.size() < 2 && !p.also) continue;
+            // the boxes of a class may start from different values
+            std::vector<Tuning> keep;
+            for (mhit_ctx* c : cls) keep.push_back(c->tune);
+            auto set = [&](int v) {   // whether that changes a box
+                bool other = false;
+                for (size_t i = 0; i < cls.size(); i++) {
+                    Tuning& t = cls[i]->tune = keep[i];
+                    other = other || t.*(p.field) != v || (p.also && t.*(p.also) != v);
+                    t.*(p.field) = v;
+                    if (p.also) t.*(p.also) = v;
                 }
+                return other;
+            };
+            int best = -1;          // none better than the current settings
+            double bms = best_ms;   // their time
+            for (int v : p.cand) {
+                if (!set(v)) continue;
                 double ms = 0.0;
                 if ((rc = trial(&ms)) != MHIT_OK) break;
                 if (ms < bms) { bms = ms; best = v; }
             }
-            for (mhit_ctx* c : cls) {
-                c->tune.*(p.field) = best;
-                if (p.also) c->tune.*(p.also) = best;
-            }
+            if (best < 0)
+                for (size_t i = 0; i < cls.size(); i++) cls[i]->tune = keep[i];
+            else
+                set(best);
             best_ms = bms;
         }
     }

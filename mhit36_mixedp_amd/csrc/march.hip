@@ -616,14 +616,13 @@ void k_acdi_march(AcdiArgs one, const AcdiArgs* __restrict__ tab, int nbox) {
 }
 
 // ------------------------------------------------------------- launchers
-// z chunk of a launch over nb boxes: the tuned one, or less where the launch
-// would then leave CUs without a workgroup (ms per step, FP32 Poisson, single
-// phase / multiphase: 32^3 0.041 / 0.061 at 4 planes -> 0.036 / 0.047 at 1,
-// 64^3 0.046 / 0.068 -> 0.042 / 0.059 at 2).
+// z chunk of a launch over nb boxes: the tuned one as it is, except that
+// kShortChunk stands for as few planes as keep the CUs busy (ms per step, FP32
+// Poisson, single phase / multiphase: 32^3 0.039 / 0.056 at 4 planes -> 0.034
+// / 0.045 at 1, 64^3 0.042 / 0.062 -> 0.038 / 0.055 at 2).
 static int pass_chunk(const mhit_ctx* c, int mz, int my, int nb) {
-    const int n = c->n, zc = n < mz ? n : mz;
-    const long long tiles = (long long)div_up(n, tile_cols(my)) * div_up(n, my) * nb;
-    return tiles * div_up(n, zc) < c->cus ? chunk_planes(n, tiles, c->cus, zc) : zc;
+    const int zc = std::min(c->n, mz);
+    return mz == kShortChunk ? busy_chunk(c->n, my, nb, zc, c->cus) : zc;
 }
 
 template <typename TD>
