@@ -136,11 +136,14 @@ void k_ns_march(NsArgs<TD> one, const NsArgs<TD>* __restrict__ tab, int nbox) {
     const int i = i0 + tx, j = j0 + ty;
     // A stopped run writes nothing; its AB2 history stays in the buffer it
     // was in, and the host undoes an odd number of buffer swaps afterwards
-    // (the finalize pass counts the skipped steps).  The flag is looked at
-    // where something is stored, as in every pass of a step: returning on it
-    // first would put its load in front of all others (about 0.6 us of each
-    // launch).
-    const bool live = i < n && j < n && !S->halted;
+    // (the finalize pass counts the skipped steps).  Every pass of a step
+    // returns before its loads: a step queued behind the stop then costs its
+    // launches and the ACDI pass's copy (256^3 multiphase 0.074 ms, 0.47 with
+    // the flag looked at only at the stores; a running step takes 0.88 either
+    // way).  No copy here: any code in this branch costs the marching loop
+    // registers.
+    if (S->halted) return;
+    const bool live = i < n && j < n;
     // global indices of the cell, or of its periodic image past the domain edge
     const int ic = wrapn(i, n), jc = wrapn(j, n);
     const double m0 = S->mean[0], m1 = S->mean[1], m2 = S->mean[2];

@@ -70,7 +70,7 @@ void k_fft_x_fwd(XFwdArgs<T> one, const XFwdArgs<T>* __restrict__ tab, int nbox)
     MHIT_GLOBAL V* __restrict__ nyq = gmem(A.nyq);
     const MHIT_GLOBAL V* __restrict__ tw = gmem(A.tw);
     const MHIT_GLOBAL DevScalars* __restrict__ S = gmem(A.S);
-    const bool halted = S && S->halted;   // looked at before the stores
+    if (S && S->halted) return;
     const int y0 = blk.x * 2 * P;
     const int z = blk.y;
     const int tid = threadIdx.x;
@@ -115,7 +115,6 @@ void k_fft_x_fwd(XFwdArgs<T> one, const XFwdArgs<T>* __restrict__ tab, int nbox)
     __syncthreads();
     fft_stages<V, N, 1, P, TPC, LD, false, N, SW, PL>(lds, tid % P, tid / P, stw);
 
-    if (halted) return;
 #pragma unroll
     for (int r = 0; r < (H * 2 * P + NT - 1) / NT; r++) {
         const int e = tid + r * NT;
@@ -170,7 +169,7 @@ void k_fft_x_inv(XInvArgs<T> one, const XInvArgs<T>* __restrict__ tab, int nbox)
     MHIT_GLOBAL T* __restrict__ pres = gmem(A.pres);
     const MHIT_GLOBAL V* __restrict__ tw = gmem(A.tw);
     const MHIT_GLOBAL DevScalars* __restrict__ S = gmem(A.S);
-    const bool halted = S && S->halted;   // looked at before the stores
+    if (S && S->halted) return;
     const int y0 = blk.x * 2 * P;
     const int z = blk.y;
     const int tid = threadIdx.x;
@@ -201,7 +200,6 @@ void k_fft_x_inv(XInvArgs<T> one, const XInvArgs<T>* __restrict__ tab, int nbox)
     __syncthreads();
     fft_stages<V, N, 1, P, TPC, LD, true, N, SW, PL>(lds, tid % P, tid / P, stw);
 
-    if (halted) return;
 #pragma unroll
     for (int r = 0; r < (N * 2 * P + NT - 1) / NT; r++) {
         const int e = tid + r * NT;
@@ -259,7 +257,7 @@ void k_fft_xy_fwd(XFwdArgs<T> one, const XFwdArgs<T>* __restrict__ tab, int nbox
     MHIT_GLOBAL V* __restrict__ nyq = gmem(A.nyq);
     const MHIT_GLOBAL V* __restrict__ tw = gmem(A.tw);
     const MHIT_GLOBAL DevScalars* __restrict__ S = gmem(A.S);
-    const bool halted = S && S->halted;   // looked at before the stores
+    if (S && S->halted) return;
     const int z = blk.y;
     const int tid = threadIdx.x;
     const int zp = (z + 1 == N) ? 0 : z + 1;
@@ -322,7 +320,6 @@ void k_fft_xy_fwd(XFwdArgs<T> one, const XFwdArgs<T>* __restrict__ tab, int nbox
     for (int r = 0; r < NSP; r++) sy[tid + r * NT] = sp[r];   // sy[y][k] at y H + k = e
     __syncthreads();
     fft_stages<V, N, 1, H, TPC, H, false>(sy, tid % H, tid / H, stw);
-    if (halted) return;
     // store spec[z][ky][kx]; kx = 0 and the Nyquist plane separated from column 0
 #pragma unroll
     for (int r = 0; r < NSP; r++) {
@@ -364,7 +361,7 @@ void k_fft_yx_inv(XInvArgs<T> one, const XInvArgs<T>* __restrict__ tab, int nbox
     MHIT_GLOBAL T* __restrict__ pres = gmem(A.pres);
     const MHIT_GLOBAL V* __restrict__ tw = gmem(A.tw);
     const MHIT_GLOBAL DevScalars* __restrict__ S = gmem(A.S);
-    const bool halted = S && S->halted;   // looked at before the stores
+    if (S && S->halted) return;
     const int z = blk.y;
     const int tid = threadIdx.x;
     stage_twiddles<V, N, NT>(stw, tw, tid);
@@ -414,7 +411,6 @@ void k_fft_yx_inv(XInvArgs<T> one, const XInvArgs<T>* __restrict__ tab, int nbox
     }
     __syncthreads();
     fft_stages<V, N, 1, P, TPC, LD, true, N, SW>(lds, tid % P, tid / P, stw);
-    if (halted) return;
 #pragma unroll
     for (int r = 0; r < N * 2 * P / NT; r++) {
         const int e = tid + r * NT;
@@ -444,7 +440,7 @@ struct ColArgs {
 // (MODE 2).
 template <typename T, int N, int C, bool AXIS_CONTIG, int MODE, bool WF>
 __device__ __forceinline__ void cols_body(const ColArgs<T>& A, const int bxi, const int byi, const bool NYQ,
-                                          const bool halted, cplx_t<T>* __restrict__ lds, cplx_t<T>* __restrict__ stw,
+                                          cplx_t<T>* __restrict__ lds, cplx_t<T>* __restrict__ stw,
                                           double* __restrict__ skk) {
     using V = cplx_t<T>;
     constexpr int TPC = FftCfg<T, N>::TPC;
@@ -605,7 +601,6 @@ __device__ __forceinline__ void cols_body(const ColArgs<T>& A, const int bxi, co
             }
             inverse();
         }
-        if (halted) return;
         if constexpr (MODE == 0) {
 #pragma unroll
             for (int r = 0; r < 8; r++) st(g + (size_t)spec_k(r) * sa + c * sc, v[r]);
@@ -672,7 +667,6 @@ __device__ __forceinline__ void cols_body(const ColArgs<T>& A, const int bxi, co
             fft_stages<V, N, NS1, C, TPC, LD, true, N / 8>(lds, c, t, stw);
             fft_last8_from_lds<V, N, LD, true>(lds, c, t, v, stw);
         }
-        if (halted) return;
 #pragma unroll
         for (int r = 0; r < 8; r++) st(elem(t * sa + c * sc, r * TPC), v[r]);
         return;
@@ -735,7 +729,6 @@ __device__ __forceinline__ void cols_body(const ColArgs<T>& A, const int bxi, co
         fft_stages<V, N, 1, C, TPC, LD, true>(lds, c, t, stw);
     }
 
-    if (halted) return;
 #pragma unroll
     for (int r = 0; r < (N * C) / NT; r++) {
         const int e = tid + r * NT;
@@ -770,7 +763,7 @@ void k_fft_cols(ColArgs<T> one, ColArgs<T> onen, const ColArgs<T>* __restrict__ 
     ColArgs<T> A = nyq ? onen : one;
     if (tab) A = nyq ? tabn[blk.box] : tab[blk.box];
     const MHIT_GLOBAL DevScalars* __restrict__ S = gmem(A.S);
-    const bool halted = S && S->halted;   // looked at before the stores
+    if (S && S->halted) return;
     const bool ac = nyq ? NYQ_AC : AC;
     const int start = nyq ? blk.nx * N : 0;                  // first workgroup of the part
     const int count = nyq ? 2 * blk.nx : blk.nx * N;
@@ -782,10 +775,10 @@ void k_fft_cols(ColArgs<T> one, ColArgs<T> onen, const ColArgs<T>* __restrict__ 
     }
     const int bxi = nyq ? L : L % blk.nx, byi = nyq ? 0 : L / blk.nx;
     if constexpr (AC == NYQ_AC) {
-        cols_body<T, N, C, AC, MODE, WF>(A, bxi, byi, nyq, halted, lds, stw, skk);   // one body for both parts
+        cols_body<T, N, C, AC, MODE, WF>(A, bxi, byi, nyq, lds, stw, skk);   // one body for both parts
     } else {
-        if (nyq) cols_body<T, N, C, NYQ_AC, MODE, WF>(A, bxi, byi, true, halted, lds, stw, skk);
-        else cols_body<T, N, C, AC, MODE, WF>(A, bxi, byi, false, halted, lds, stw, skk);
+        if (nyq) cols_body<T, N, C, NYQ_AC, MODE, WF>(A, bxi, byi, true, lds, stw, skk);
+        else cols_body<T, N, C, AC, MODE, WF>(A, bxi, byi, false, lds, stw, skk);
     }
 }
 

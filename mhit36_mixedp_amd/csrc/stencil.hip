@@ -317,7 +317,7 @@ void k_correct(CorrArgs<T> one, const CorrArgs<T>* __restrict__ tab, int nbox) {
     xcd_tile(tbx, tby, tbz, blk, A.xcd);
     const int i = tbx * MX + threadIdx.x, j = tby * MY + threadIdx.y;
     const int z0 = tbz * A.zc, z1 = min(z0 + A.zc, n);
-    const bool halted = S->halted;       // looked at before the stores
+    if (S->halted) return;               // the finalize pass reads no partials then
     const double dtr = g.dt / g.rho;
     double su = 0.0, sv = 0.0, sw = 0.0;
     double mu_ = -INFINITY, mv_ = -INFINITY, mw_ = -INFINITY;
@@ -344,7 +344,7 @@ void k_correct(CorrArgs<T> one, const CorrArgs<T>* __restrict__ tab, int nbox) {
                 const double uu = uq[t] - dtr * (c - (double)px[t]) * g.dxi;
                 const double vv = vq[t] - dtr * (c - (double)py[t]) * g.dxi;
                 const double ww = wq[t] - dtr * (c - (double)pm) * g.dxi;
-                if (!halted) { st_once(&u[q], uu); st_once(&v[q], vv); st_once(&w[q], ww); }
+                st_once(&u[q], uu); st_once(&v[q], vv); st_once(&w[q], ww);
                 su += uu; sv += vv; sw += ww;
                 mu_ = fmax(mu_, uu); mv_ = fmax(mv_, vv); mw_ = fmax(mw_, ww);
                 pm = pc[t];
@@ -519,7 +519,7 @@ void k_fin_rows(FinArgs one, const FinArgs* __restrict__ tab) {
     FinArgs A = one;
     if (tab) A = tab[blockIdx.y];
     const int q = blockIdx.x * 256 + threadIdx.x, t = q / 6, f = q - 6 * t;
-    if (t >= A.nparts) return;
+    if (t >= A.nparts || gmem(A.S)->halted) return;
     MHIT_GLOBAL double* partials = gmem(A.partials);
     const int nx = A.g.n / 64, tiles = A.nblocks / 8;
     double r = f < 3 ? 0.0 : -INFINITY;
@@ -533,7 +533,7 @@ void k_fin_rows(FinArgs one, const FinArgs* __restrict__ tab) {
         for (int j = 1; j < 8; j++) x[0] = f < 3 ? x[0] + x[j] : fmax(x[0], x[j]);
         r = f < 3 ? r + x[0] : fmax(r, x[0]);
     }
-    if (!gmem(A.S)->halted) partials[(size_t)(A.nblocks + t) * 6 + f] = r;
+    partials[(size_t)(A.nblocks + t) * 6 + f] = r;
 }
 
 // One workgroup per box (blockIdx.x is the box of a batched launch).
@@ -547,7 +547,10 @@ void k_finalize(FinArgs one, const FinArgs* __restrict__ tab) {
     const int nblocks = A.nparts ? A.nparts : A.nblocks;
     __shared__ double red[6][512];
     const int t = threadIdx.x;
-    const bool halted = S->halted;     // partials of a stopped run are not used
+    if (S->halted) {
+        if (t == 0) S->skipped += 1;   // a step whose passes all returned at once
+        return;
+    }
     double a[6] = {0.0, 0.0, 0.0, -INFINITY, -INFINITY, -INFINITY};
     for (int b = t; b < nblocks; b += 1024) {
         for (int f = 0; f < 3; f++) a[f] += partials[(size_t)b * 6 + f];
@@ -569,8 +572,7 @@ void k_finalize(FinArgs one, const FinArgs* __restrict__ tab) {
             const double x = __shfl_down(a[f], s, 64);
             a[f] = f < 3 ? a[f] + x : fmax(a[f], x);
         }
-    if (t == 0 && halted) S->skipped += 1;   // a step that stored nothing
-    if (t == 0 && !halted) {
+    if (t == 0) {
         const double nn = (double)g.n;
         double m[3], mx[3];
         for (int f = 0; f < 3; f++) {

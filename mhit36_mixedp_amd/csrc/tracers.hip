@@ -66,7 +66,7 @@ void k_tracers(const double* __restrict__ u, const double* __restrict__ v, const
                double* __restrict__ px, double* __restrict__ py, double* __restrict__ pz,
                double* __restrict__ pu1, double* __restrict__ pv1, double* __restrict__ pw1,
                long long np, Grid g, const DevScalars* __restrict__ S) {
-    const bool halted = S->halted;   // looked at before the stores
+    if (S->halted) return;
     const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= np) return;
     const double m[3] = {S->mean[0], S->mean[1], S->mean[2]};
@@ -88,7 +88,6 @@ void k_tracers(const double* __restrict__ u, const double* __restrict__ v, const
     x = x - lx * (double)(int)floor(x / lx);
     y = y - lx * (double)(int)floor(y / lx);
     z = z - lx * (double)(int)floor(z / lx);
-    if (halted) return;
     px[p] = x; py[p] = y; pz[p] = z;
     pu1[p] = up; pv1[p] = vp; pw1[p] = wp;
 }
