@@ -54,12 +54,13 @@ struct Tuning {
     int ac_mz = 64;       // planes per workgroup, ACDI pass (likewise)
     int xcd = 0;          // XCD-aware tile order (mhit_create: 1 up to 256^3
                           // and for boxes batched in an ensemble, 0 above)
-    int sort_every = 32;  // steps between tracer re-orderings (0: never).  At a
-                          // CFL number near 0.01, us per step every 10 / 20 /
-                          // 40 / 160 steps / never: 32^3 with 1000 tracers 42.3
-                          // / 40.4 / 39.6 / 39.2 / 39.4, 256^3 with 1M 724 / 717
-                          // / 716 / 726 / 744, 512^3 with 4M 5268 / 5249 / 5244
-                          // / 5294 / 5376
+    int sort_every = 32;  // steps between tracer re-orderings (0: never).  us
+                          // per step every 10 / 32 / 64 steps, single phase:
+                          // CFL number 0.01 32^3 with 1000 tracers 42.0 / 39.8
+                          // / 39.3, 256^3 with 1M 673 / 665 / 664, 512^3 with
+                          // 4M 5026 / 4999 / 4997; CFL number 0.35 256^3 679 /
+                          // 671 / 670, 384^3 with 2M 2294 / 2272 / 2270, 512^3
+                          // 5031 / 5000 / 4990
     int ns_my = 16;       // tile rows, NS pass: 16 or 8 (64 columns), 32 (32
                           // columns) or 10 (96 columns); mhit_create: 8 for
                           // n <= 64, 10 where n is a multiple of 96 but not
