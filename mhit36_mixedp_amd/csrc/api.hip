@@ -147,10 +147,10 @@ int busy_chunk(int n, int my, int nb, int zc, int cus) {
 }
 
 // Launch shapes by grid size, then MHIT_TUNE; mhit_autotune refines.
-// A box alone: 64 x 8 tiles up to 64^3, 64 x 16 above (less halo), and
-// 64 x 8 in the ACDI pass below 256^3, two workgroups to a CU (against
-// 64 x 16, ms per step: 128^3 0.147 and 0.147, 192^3 0.450 and 0.452; from
-// 256^3 the halo costs more: 0.823 and 0.802, 384^3 2.82 and 2.82); z chunks
+// A box alone: 64 x 8 tiles up to 64^3, 64 x 16 above (less halo; 64 x 8 in
+// the ACDI pass, two workgroups to a CU, measured the same at 128^3 and 192^3,
+// 145.4 and 145.4 us, 401 and 402 us per step, FP64 155.8 and 155.3, 448 and
+// 448, and slower at 256^3, 0.823 against 0.802 ms); z chunks
 // by chunk_planes.  Measured, ms per step, FP32
 // Poisson, single phase / multiphase, against chunks halved from
 // min(128, n/4) until there is a workgroup per CU: 96^3 0.081 / 0.114 at 6
@@ -175,11 +175,8 @@ void default_tuning(mhit_ctx* c, bool batched, bool env) {
     c->tune.ac_my = rows;
     c->tune.ns_mz = c->tune.ac_mz = std::min(128, n);
     if (!batched) {
-        if (rows == 16 && n < 256) c->tune.ac_my = 8;
-        auto tiles = [&](int my) { return (long long)div_up(n, tile_cols(my)) * div_up(n, my); };
-        const int ac_slots = (c->tune.ac_my == 8 && n > 64) ? 2 * c->cus : c->cus;
-        c->tune.ns_mz = std::max(kShortChunk, chunk_planes(n, tiles(rows), c->cus, 256));
-        c->tune.ac_mz = std::max(kShortChunk, chunk_planes(n, tiles(c->tune.ac_my), ac_slots, 256));
+        const long long tiles = (long long)div_up(n, tile_cols(rows)) * div_up(n, rows);
+        c->tune.ns_mz = c->tune.ac_mz = std::max(kShortChunk, chunk_planes(n, tiles, c->cus, 256));
     }
     // XCD tile order: neighbouring tiles of a box then share an XCD's L2.
     // Batched (the 64^3 / 96^3 / 128^3 ensemble 18.78-18.84k -> 18.87-

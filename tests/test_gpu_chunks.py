@@ -56,3 +56,25 @@ def test_ensemble_reports_the_chunks_it_launches():
                     print(n, phase, mz, t[mz], tiles * -(-n // t[mz]), flush=True)
                     assert all(g[mz] == t[mz] for g in group)
                     assert t[mz] == 1 or tiles * -(-n // t[mz]) >= 0.8 * cus
+
+
+@pytest.mark.parametrize("n,prec", [(128, 1), (192, 0)])
+def test_both_passes_share_a_shape_above_64(n, prec):
+    """Above 64^3 the ACDI pass has the tiles and chunks of the NS pass by
+    default, and the bits of 64 x 8 tiles."""
+    import numpy as np
+    from mhit36_mixedp_amd import Solver
+    print(f"[chunks] shared shape n={n}", flush=True)
+    phi = []
+    for shape in ({}, dict(ac_my=8, ac_mz=19)):
+        with Solver(nx=n, phiflag=1, sigma=0.5, dt=2e-4, poisson_precision=prec) as s:
+            t = s.tuning()
+            assert t["ac_my"] == t["ns_my"] == 16 and t["ac_mz"] == t["ns_mz"]
+            if shape:
+                s.set_tuning(**shape)
+            s.init_random_velocity(5, kmax=4.0, urms=1.0)
+            s.init_drops(1, 1.2, 5)
+            s.step(3)
+            phi.append((s.download_field(5), s.download_field(9)))
+    for a, b in zip(*phi):
+        assert np.array_equal(a, b)
