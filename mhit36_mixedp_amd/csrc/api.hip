@@ -127,7 +127,7 @@ static void parse_tuning(const char* s, Tuning& t) {
 // `slots`, and each costs its planes plus about four for the planes before
 // and after it, so rounds x (planes + 4) is what the last workgroup waits
 // for; the longest of equal choices has the least halo.
-int chunk_planes(int n, long long tiles, int slots, int cap) {
+static int chunk_planes(int n, long long tiles, int slots, int cap) {
     int best = 1;
     long long cost = -1;
     for (int c = 1; c <= n; c++) {

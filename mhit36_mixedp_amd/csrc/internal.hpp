@@ -214,11 +214,8 @@ double* state_field(mhit_ctx* c, int fieldn);
 // ensemble), then the MHIT_TUNE overrides
 void default_tuning(mhit_ctx* c, bool batched, bool env = true);
 void tuning_env(mhit_ctx* c);   // the MHIT_TUNE overrides alone
-// api.hip: planes per workgroup (at most cap) of a marching pass over
-// `tiles` tiles, `slots` workgroups resident at once
-int chunk_planes(int n, long long tiles, int slots, int cap);
-// zc planes per workgroup of a pass over nb boxes in tiles of `my` rows, or
-// fewer where CUs would idle
+// api.hip: zc planes per workgroup of a pass over nb boxes in tiles of `my`
+// rows, or fewer where CUs would idle
 int busy_chunk(int n, int my, int nb, int zc, int cus);
 // dump.hip: wait for a pending dump and free its buffers
 void dump_release(mhit_ctx* c);

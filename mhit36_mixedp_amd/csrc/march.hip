@@ -18,6 +18,7 @@
 // each intermediate lives changes.
 #include "internal.hpp"
 
+#include <algorithm>
 #include <type_traits>
 #include <vector>
 
@@ -111,8 +112,8 @@ void k_ns_march(NsArgs<TD> one, const NsArgs<TD>* __restrict__ tab, int nbox) {
     // ABC forcing by row and column of the tile (main.f90:711-713): f2 cos y,
     // f2 sin y, f1 sin x, f1 cos x.  Read from the global tables inside the
     // plane loop they queued behind the next plane's loads, so that every
-    // plane waited for the plane after it: 512^3 multiphase 2.95 -> 2.68 ms
-    // (6.4 TB/s of counted traffic), 256^3 0.380 -> 0.337, single phase 384^3
+    // plane waited for the plane after it: 512^3 multiphase 2.95 -> 2.71 ms
+    // (6.3 TB/s of counted traffic), 256^3 0.380 -> 0.337, single phase 384^3
     // 1.11 -> 1.05.
     __shared__ double scy[MY], ssy[MY], ssx[MX], scx[MX];
 
@@ -384,8 +385,8 @@ void k_ns_march(NsArgs<TD> one, const NsArgs<TD>* __restrict__ tab, int nbox) {
 // Lanes without a cell of their own store to the kSink elements behind the
 // field, and a chunk fetches one plane that it does not use.  Before, with
 // stores and loads under conditions, each plane waited for all of them: ms
-// with / without conditions (FP32 Poisson, multiphase) 512^3 1.68 / 1.43
-// (5.3 TB/s of counted traffic), 256^3 0.220 / 0.198, 192^3 0.100 / 0.087, 128^3
+// with / without conditions (FP32 Poisson, multiphase) 512^3 1.68 / 1.45
+// (5.8 TB/s of counted traffic), 256^3 0.220 / 0.198, 192^3 0.100 / 0.087, 128^3
 // 0.0370 / 0.0344, 96^3 0.0238 / 0.0235.  The 32-bit offsets took the kernel
 // from 124 to 96 registers.
 

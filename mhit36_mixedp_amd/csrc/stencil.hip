@@ -255,9 +255,10 @@ int launch_ns(mhit_ctx* c) {
 // 256^3 its workgroups are wide and flat, so that the dispatch order sweeps
 // memory front to back.  FP64: 128 x 4 columns of two planes, 512^3 1.36 ->
 // 1.18 ms (6.3 TB/s).  FP32: rows of 256 cells (128 x 2 where n is no
-// multiple of 256) over the order's chunk, 512^3 1.27 -> 1.22 ms, 384^3 0.59
+// multiple of 256) over the order's chunk, 512^3 1.27 -> 1.20 ms, 384^3 0.59
 // -> 0.54, 256^3 0.172 -> 0.158 (5.5 TB/s) against the march; a wave writes
-// its row's sums and k_fin_rows (4 us) adds them up as an 8-row tile would.
+// its row's sums and k_fin_rows (5 us at 256^3 and 384^3, 11 at 512^3) adds
+// them up as an 8-row tile would.
 // The rows start where a launch covers as many cells as 256^3, so that an
 // ensemble's batches of 128^3 take them too (eight planes in flight: 16 x
 // 64^3 + 16 x 96^3 + 16 x 128^3 2.44 -> 2.36 ms per step, 16 x 128^3 1.51 ->
